@@ -69,6 +69,7 @@ struct StepArgs {
     // each halo plane (the launch covers 2 * part_edge along part_axis); 2 the others (the launch
     // covers n - 2 * part_edge).  part_axis: 1 the halo axis is ax1, 2 it is ax2.
     int part, part_axis, part_edge;
+    int store_end;         // last column stored in a row (Layout::row_store_end)
 };
 
 // Signed sum  sx*a + sy*b + sz*c  for compile-time signs in {-1,0,1}: adds only.  With no term the
@@ -166,11 +167,12 @@ __host__ __device__ __forceinline__ CellAux<R> cell_aux(const StepArgs<R>& a, in
 }
 
 // AUX: the per-cell inputs come from aux (read ahead by the caller); otherwise they are read here
-// where they are used.
+// where they are used.  sums: add the cell to the averaging sums if those are on (false in a lane
+// that repeats another's cell).
 template <int Q, class C, bool BGK3, bool HRR, bool VRE, bool AUX = false>
 __host__ __device__ __forceinline__ void collide_cell(const StepArgs<typename C::real>& a, const typename C::raw (&rv)[Q],
                                                       const CellAux<typename C::real>& aux, int i, int j, int k, int ca,
-                                                      int cb, int cc, int oc, typename C::real (&dev)[Q],
+                                                      int cb, int cc, int oc, bool sums, typename C::real (&dev)[Q],
                                                       typename C::real& tau_out) {
     using R = typename C::real;
     using Lt = Lattice<Q>;
@@ -216,7 +218,7 @@ __host__ __device__ __forceinline__ void collide_cell(const StepArgs<typename C:
     R rh = R(1) + dr;
     const R invrho = recip(rh);
     R ux = (jx * invS) * invrho, uy = (jy * invS) * invrho, uz = (jz * invS) * invrho;
-    if (a.avg != nullptr) {
+    if (a.avg != nullptr && sums) {
         // time averaging of the moments after the previous step (src/m_averaging_full_kernel.F90:33-39)
         // (the six sums are read before any is written: one memory round trip instead of six)
         R* p = a.avg + oc;
@@ -418,7 +420,7 @@ template <int Q, class C, bool BGK3, bool HRR, bool VRE>
 __host__ __device__ __forceinline__ void collide_cell(const StepArgs<typename C::real>& a, const typename C::raw (&rv)[Q], int i,
                                                       int j, int k, int ca, int cb, int cc, int oc,
                                                       typename C::real (&dev)[Q], typename C::real& tau_out) {
-    collide_cell<Q, C, BGK3, HRR, VRE, false>(a, rv, CellAux<typename C::real>{}, i, j, k, ca, cb, cc, oc, dev, tau_out);
+    collide_cell<Q, C, BGK3, HRR, VRE, false>(a, rv, CellAux<typename C::real>{}, i, j, k, ca, cb, cc, oc, true, dev, tau_out);
 }
 
 // The closed-face pass of axis D (src/m_boundary_{i,j,k}_closed_kernel.F90) performed by the
@@ -579,8 +581,9 @@ __device__ __forceinline__ void buffer_store(void* base, int nbytes, uint32_t vo
 }
 #endif
 
-// One cell of the step at storage coordinates (ca, cb, cc) (1-based along ax0, ax1, ax2):
-// gather the streamed populations, collide, store, and the folded face pass.
+// One cell of the step at storage coordinates (cs, cb, cc) (1-based along ax0, ax1, ax2):
+// gather the streamed populations, collide, store, and the folded face pass.  Columns cs past the
+// row's last cell, up to store_end, store that cell's populations (Layout::row_store_end).
 // VAR bit 0: non-temporal stores, bit 1: non-temporal loads (measured slower; kept for tuning),
 // bit 3: the buffer is below 4 GiB (32-bit offsets from one base), bit 4: row-blocked buffers of
 // any size addressed per slab of the slowest axis (one scalar base per source slab, 32-bit offsets
@@ -589,12 +592,14 @@ __device__ __forceinline__ void buffer_store(void* base, int nbytes, uint32_t vo
 // make_layout's order), so i, j, k map to (ca, cb, cc) without run-time selects, and the caller's
 // wave-uniform cb, cc keep the row's offsets, wraps and checks in scalar registers.
 template <int Q, class C, bool BGK3, bool HRR, bool VRE, int VAR, int AXS = -1>
-__device__ __forceinline__ void step_cell(const StepArgs<typename C::real>& a, int ca, int cb, int cc) {
+__device__ __forceinline__ void step_cell(const StepArgs<typename C::real>& a, int cs, int cb, int cc) {
     using R = typename C::real;
     using raw = typename C::raw;
     using Lt = Lattice<Q>;
     const Layout& L = a.lay;
-    if (ca > L.n(L.ax0) || cb > L.n(L.ax1) || cc > L.n(L.ax2)) return;
+    if (cs > a.store_end || cb > L.n(L.ax1) || cc > L.n(L.ax2)) return;
+    const int n0 = L.n(L.ax0);
+    const int ca = cs < n0 ? cs : n0;
     int i, j, k;
     constexpr int A1 = AXS == 0 ? 1 : 0, A2 = AXS == 2 ? 1 : 2;
     if constexpr (AXS < 0) {
@@ -676,7 +681,7 @@ __device__ __forceinline__ void step_cell(const StepArgs<typename C::real>& a, i
     const int (&d2)[3] = A2 == 0 ? ox : A2 == 1 ? oy : oz;
     const int w0 = SLAB ? oc0 - cc * s2 : 0;      // cell offset within its slab
     const size_t slab0 = SLAB ? (size_t)cc * (size_t)s2 : 0;
-    const int sbytes = (int)((uint32_t)s2 * (uint32_t)sizeof(raw));
+    const int sbytes = (int)(((uint32_t)s2 + (uint32_t)line_elems(sizeof(raw))) * (uint32_t)sizeof(raw));
 #pragma unroll
     for (int l = 0; l < Q; ++l) {
         if constexpr (SLAB) {
@@ -705,8 +710,8 @@ __device__ __forceinline__ void step_cell(const StepArgs<typename C::real>& a, i
 
     R out[Q];
     R tau = 0;
-    const int oc = oc0;
-    collide_cell<Q, C, BGK3, HRR, VRE, AUX>(a, rv, aux, i, j, k, ca, cb, cc, occ, out, tau);
+    const int oc = oc0 + (cs - ca);   // unit stride along ax0
+    collide_cell<Q, C, BGK3, HRR, VRE, AUX>(a, rv, aux, i, j, k, ca, cb, cc, occ, cs == ca, out, tau);
 
     char* __restrict__ dstb = static_cast<char*>(a.dst);
     const uint32_t ob = (uint32_t)oc * (uint32_t)sizeof(raw);
@@ -714,7 +719,7 @@ __device__ __forceinline__ void step_cell(const StepArgs<typename C::real>& a, i
     for (int l = 0; l < Q; ++l) {
         if constexpr (SLAB) {
 #if defined(__HIP_DEVICE_COMPILE__)
-            buffer_store<raw, (VAR & 1) != 0>(dstb + slab0 * sizeof(raw), sbytes, (uint32_t)w0 * (uint32_t)sizeof(raw),
+            buffer_store<raw, (VAR & 1) != 0>(dstb + slab0 * sizeof(raw), sbytes, (uint32_t)(w0 + (cs - ca)) * (uint32_t)sizeof(raw),
                                               (uint32_t)l * pb32, C::template enc_dep<Q>(out[l], l));
 #endif
             continue;
@@ -731,6 +736,7 @@ __device__ __forceinline__ void step_cell(const StepArgs<typename C::real>& a, i
         if constexpr ((VAR & 1) != 0) __builtin_nontemporal_store(C::template enc_dep<Q>(out[l], l), p);
         else *p = C::template enc_dep<Q>(out[l], l);
     }
+    if (cs != ca) return;
     if (VRE && a.tau_out != nullptr) a.tau_out[occ] = tau;
     if (a.fold_dir >= 0) fold_closed_face<Q, C>(a, i, j, k, out);
     if (a.inflow_fold && (i == 1 || i == L.nx)) fold_inflow<Q, C>(a, i, j, k, out);

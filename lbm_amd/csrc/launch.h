@@ -129,6 +129,7 @@ struct Launch {
         a.part = h.part;
         a.part_axis = h.part_axis;
         a.part_edge = h.part_edge;
+        a.store_end = L.row_store_end((int)sizeof(typename C::raw));
         return a;
     }
 

@@ -1,14 +1,20 @@
 // Device layout of one population buffer.
 //
 // Cells of the padded grid (0:nx+1, 0:ny+1, 0:nz+1) lie in rows along one axis (the "fast" axis);
-// rows are padded so that interior index 1 starts on a 128-byte boundary (storage column of index
-// x is xoff + x with xoff = 128/sizeof(raw) - 1) and the row pitch is a multiple of 128 bytes.
+// interior index 1 starts on a 128-byte boundary and the row pitch is the smallest multiple of 128
+// bytes that holds a row's n + 2 cells.  Ghost 0 of a row is the last element of the row before it
+// (behind that row's ghost n + 1); one line before the first row holds the first row's.  A line of
+// its own for that one ghost (the pitch before) left a quarter of the buffer's 256-byte blocks
+// untouched at 192 cells of 4 bytes and a third at 96; measured on MI355X with the smaller pitch,
+// D3Q27 FP32: rows of 192 cells 356 -> 352 us (384x192x128), rows of 200 453 -> 431 us
+// (384x200x128); D3Q19 FP32 rows of 96 55.4 -> 52.8 us (192x96x96).  Pitches of 64- or 32-byte
+// multiples, whose rows no longer start on lines, measured 382 and 449 us at 192 cells.
 // The two other axes follow in natural order.  A 64-lane wave along the fast axis reads and
 // writes whole cache lines for populations with no velocity along that axis.
 //
 // Two arrangements of the Q populations, both addressed as  l * plane + cell(i, j, k):
 //   row-blocked (the default; needs element offsets below 2^31 and one slab of the slowest axis
-//     below 4 GiB): [row][population][pitch] - plane is the row pitch and the row strides are Q
+//     and a line below 4 GiB): [row][population][pitch] - plane is the row pitch and the row strides are Q
 //     times larger; the Q segments of a row are adjacent;
 //   planes: [population][row][pitch] - plane is the whole padded grid.
 // Per-cell arrays (tau, moments, forcing, averages) always use the plane arrangement of one
@@ -54,6 +60,17 @@ struct Layout {
     __host__ __device__ inline int cell_w(int i, int j, int k) const {
         return cell(wrap(i, nx, per_i), wrap(j, ny, per_j), wrap(k, nz, per_k));
     }
+    // Last column (index along ax0) that the step kernel stores in an interior row: with a periodic
+    // ax0 its lanes past the row's end fill the last 64 bytes with copies of the row's last cell, in
+    // columns that hold nothing (the ghosts of a periodic axis are not read).  A row whose end leaves
+    // 64 bytes partly written costs a read of them: measured on MI355X, rows of 200 cells, D3Q27 FP16
+    // 400x200x100 198 -> 182 us, FP32 384x200x128 431 -> 416 us; whole lines instead of 64 bytes gain
+    // nothing more (FP16 200 us, 97x95x96 FP32 44.0 -> 47.0 us).
+    __host__ __device__ inline int row_store_end(int raw_bytes) const {
+        const int n0 = n(ax0), g = 64 / raw_bytes;
+        const int per = ax0 == 0 ? per_i : ax0 == 1 ? per_j : per_k;
+        return per ? (n0 + g - 1) / g * g : n0;
+    }
     // Map coordinates given in storage-axis order (a along ax0, b along ax1, c along ax2) to i,j,k.
     __host__ __device__ inline void ijk(int a, int b, int c, int& i, int& j, int& k) const {
         i = ax0 == 0 ? a : (ax1 == 0 ? b : c);
@@ -70,9 +87,12 @@ __host__ __device__ inline int part_row(int c, int part, int n, int e) {
     return part == 1 ? (c < e ? c : c < 2 * e ? n - 2 * e + c : n) : (c < n - 2 * e ? c + e : n);
 }
 
+// Elements of a 128-byte line.
+__host__ __device__ inline constexpr int line_elems(int raw_bytes) { return 128 / raw_bytes; }
+
 // fast < 0: choose (first periodic axis, else i).  q > 0 with rowblock: row-blocked buffers when every
-// element offset fits 31 bits and one slab of the slowest axis (Q rows per ax1 index) stays below
-// 4 GiB (the step kernel's 32-bit offsets within a slab), planes otherwise.
+// element offset fits 31 bits and one slab of the slowest axis (Q rows per ax1 index) and the line
+// behind it stay below 4 GiB (the step kernel's 32-bit offsets within a slab), planes otherwise.
 inline Layout make_layout(int nx, int ny, int nz, int raw_bytes, int per_i, int per_j, int per_k, int fast = -1,
                           int q = 0, bool rowblock = false) {
     Layout L;
@@ -82,9 +102,9 @@ inline Layout make_layout(int nx, int ny, int nz, int raw_bytes, int per_i, int 
     L.ax0 = fast;
     L.ax1 = fast == 0 ? 1 : 0;
     L.ax2 = fast == 2 ? 1 : 2;
-    const int a = 128 / raw_bytes;           // elements per 128 B
+    const int a = line_elems(raw_bytes);
     const int n0 = L.n(L.ax0), n1 = L.n(L.ax1), n2 = L.n(L.ax2);
-    L.pitch = ((a + n0 + 1) + a - 1) / a * a;
+    L.pitch = (n0 + 2 + a - 1) / a * a;
     int st[3];
     st[L.ax0] = 1;
     st[L.ax1] = L.pitch;
@@ -93,15 +113,15 @@ inline Layout make_layout(int nx, int ny, int nz, int raw_bytes, int per_i, int 
     L.base = a - 1;
     const long long pl = (long long)L.pitch * (n1 + 2) * (n2 + 2);
     const long long ea = 256 / raw_bytes;
-    L.cplane = (pl + ea - 1) / ea * ea;
+    L.cplane = (pl + a + ea - 1) / ea * ea;
     const int nq = q > 0 ? q : 1;
     L.rowblock = rowblock && q > 0 && (double)nq * (double)L.cplane < 2147483648.0 &&
-                 (double)nq * L.pitch * (n1 + 2) * raw_bytes < 4294967296.0;
+                 ((double)nq * L.pitch * (n1 + 2) + a) * raw_bytes < 4294967296.0;
     if (L.rowblock) {
         st[L.ax1] = nq * L.pitch;
         st[L.ax2] = nq * L.pitch * (n1 + 2);
         L.plane = L.pitch;
-        L.total = (nq * pl + ea - 1) / ea * ea;
+        L.total = (nq * pl + a + ea - 1) / ea * ea;
     } else {
         L.plane = L.cplane;
         L.total = nq * L.cplane;

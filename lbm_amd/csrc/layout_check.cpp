@@ -5,7 +5,9 @@
 //   * per-cell indices are distinct and inside cplane;
 //   * row-blocked buffers are chosen only while element offsets fit 31 bits and a slab of the
 //     slowest axis is below 4 GiB, and every element of a slab lies within [slab start, slab
-//     start + slab stride), the range of the step kernel's per-slab 32-bit offsets;
+//     start + slab stride + one line), the range of the step kernel's per-slab 32-bit offsets;
+//   * the columns that the step kernel's padding lanes store to lie inside that range and inside
+//     the buffer, and hold no interior cell and no ghost cell of another axis;
 //   * the two launches of a split step (part_row) cover every cell of the halo axis exactly once
 //     and map every other launch coordinate past the last cell, for any block height.
 // Prints one JSON line per case; exits non-zero on the first violation.
@@ -38,10 +40,37 @@ static int check(int nx, int ny, int nz, int raw, int q, int pi, int pj, int pk,
                         const int a2 = L.ax2 == 0 ? i : L.ax2 == 1 ? j : k;
                         const long long s2 = L.ax2 == 0 ? L.si : L.ax2 == 1 ? L.sj : L.sk;
                         const long long w = e - (long long)a2 * s2;
-                        if (w < 0 || w >= s2) return 9;
+                        if (w < 0 || w >= s2 + line_elems(raw)) return 9;
                     }
                 }
             }
+    // padding columns n0 + 1 .. row_store_end: they may overlap ghosts of the (periodic) contiguous
+    // axis, which no kernel reads, and nothing else
+    const int n0 = L.n(L.ax0);
+    const int per0 = L.ax0 == 0 ? pi : L.ax0 == 1 ? pj : pk;
+    const int end = L.row_store_end(raw);
+    if (end < n0 || (!per0 && end != n0)) return 10;
+    std::vector<unsigned char> used((size_t)L.total, 0);
+    if (end > n0)
+        for (int c = 0; c <= L.n(L.ax2) + 1; ++c)
+            for (int b = 0; b <= L.n(L.ax1) + 1; ++b)
+                for (int a = 1; a <= n0; ++a)
+                    for (int l = 0; l < q; ++l) {
+                        int i, j, k;
+                        L.ijk(a, b, c, i, j, k);
+                        used[(size_t)((long long)l * L.plane + L.cell(i, j, k))] = 1;
+                    }
+    for (int c = 1; end > n0 && c <= L.n(L.ax2); ++c)
+        for (int b = 1; b <= L.n(L.ax1); ++b)
+            for (int a = n0 + 1; a <= end; ++a)
+                for (int l = 0; l < q; ++l) {
+                    int i, j, k;
+                    L.ijk(n0, b, c, i, j, k);
+                    const long long e = (long long)l * L.plane + L.cell(i, j, k) + (a - n0);
+                    if (e >= L.total || used[(size_t)e]) return 11;
+                    const long long s2 = L.ax2 == 0 ? L.si : L.ax2 == 1 ? L.sj : L.sk;
+                    if (L.rowblock && e - c * s2 >= s2 + line_elems(raw)) return 12;
+                }
     if (L.rowblock && ((double)L.total >= 2147483648.0 ||
                        (double)(L.ax2 == 0 ? L.si : L.ax2 == 1 ? L.sj : L.sk) * raw >= 4294967296.0))
         return 4;
