@@ -16,6 +16,7 @@
 #include "../../include/lbm_hip.h"
 #include "ctx.h"
 #include "dual.h"
+#include "fields.h"
 #include "impl.h"
 #include "layout.h"
 
@@ -246,13 +247,16 @@ int lbm_adjoint_run(lbm_ctx* c, int it0, int nsteps, int every, const int32_t* b
         }
         // results
         double s = 0.0;
-        std::vector<double> hs((size_t)d.ny * d.nz), hf, ha(2 * (size_t)nblk);
+        std::vector<double> hs((size_t)d.ny * d.nz), ha(2 * (size_t)nblk);
+        const size_t gbytes = 3 * ncell_padded(c) * sizeof(double);
+        if (gFp) {
+            // the gradient in the reference's layout
+            if (int r = dev_alloc(c, c->stage, gbytes)) return r;
+            HIPCHK(c, (cells_out<3, true>(c->lay, GradientOut{gFp}, static_cast<double*>(c->stage.p), c->stream)));
+            HIPCHK(c, hipMemcpyAsync(grad_force, c->stage.p, gbytes, hipMemcpyDeviceToHost, c->stream));
+        }
         HIPCHK(c, hipMemcpyAsync(ha.data(), acc.p, ha.size() * sizeof(double), hipMemcpyDeviceToHost, c->stream));
         HIPCHK(c, hipMemcpyAsync(hs.data(), gS.p, hs.size() * sizeof(double), hipMemcpyDeviceToHost, c->stream));
-        if (gFp) {
-            hf.resize(3 * plane);
-            HIPCHK(c, hipMemcpyAsync(hf.data(), gFp, hf.size() * sizeof(double), hipMemcpyDeviceToHost, c->stream));
-        }
         HIPCHK(c, hipStreamSynchronize(c->stream));
         for (int q = 0; q < nblk; ++q) s += ha[2 * q];
         *J = s * kappa;
@@ -262,20 +266,7 @@ int lbm_adjoint_run(lbm_ctx* c, int it0, int nsteps, int every, const int32_t* b
                 for (int j = 0; j < d.ny; ++j) t += hs[(size_t)k * d.ny + j];
                 grad_shear[k] = t;
             }
-        if (grad_force) {
-            const size_t nxp = d.nx + 2, nyp = d.ny + 2, nzp = d.nz + 2;
-            std::fill(grad_force, grad_force + 3 * nxp * nyp * nzp, 0.0);
-            if (gFp)
-                for (int k = 1; k <= d.nz; ++k)
-                    for (int j = 1; j <= d.ny; ++j)
-                        for (int i = 1; i <= d.nx; ++i) {
-                            const size_t o = c->lay.cidx(i, j, k);
-                            double* g = grad_force + 3 * ((k * nyp + j) * nxp + i);
-                            g[0] = hf[o];
-                            g[1] = hf[plane + o];
-                            g[2] = hf[2 * plane + o];
-                        }
-        }
+        if (grad_force && !gFp) std::fill(grad_force, grad_force + 3 * ncell_padded(c), 0.0);
         return LBM_OK;
     };
     return run();

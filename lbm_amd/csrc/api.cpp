@@ -619,8 +619,8 @@ int lbm_init_equilibrium(lbm_ctx* c, const void* rho, const void* u, const void*
     HIPCHK(c, hipMemcpyAsync(st + 2 * cb, v, cb, hipMemcpyHostToDevice, c->stream));
     HIPCHK(c, hipMemcpyAsync(st + 3 * cb, w, cb, hipMemcpyHostToDevice, c->stream));
     // fB = feq with clamped ghosts; fA = fB; boundarycond(fB,fA); boundarycond(fA,fB)
-    HIPCHK(c, c->ops->feq_init(c->lay, c->d.ibgk == 3, st, st + cb, st + 2 * cb, st + 3 * cb, realkind, c->buf[1],
-                               c->ext[0].p, c->ext[1].p, c->ext[2].p, c->ext[3].p, c->stream));
+    void* const ext[4] = {c->ext[0].p, c->ext[1].p, c->ext[2].p, c->ext[3].p};
+    HIPCHK(c, c->ops->feq_init(c->lay, c->d.ibgk == 3, st, realkind, c->buf[1], ext, c->stream));
     HIPCHK(c, hipMemcpyAsync(c->buf[0], c->buf[1], c->buf_bytes, hipMemcpyDeviceToDevice, c->stream));
     if (int rc = boundary(c, c->buf[1], c->buf[0], it0)) return rc;
     if (int rc = boundary(c, c->buf[0], c->buf[1], it0)) return rc;
@@ -792,50 +792,21 @@ int lbm_get_averages(lbm_ctx* c, void* uave, void* vave, void* wave, void* ti, i
     if (int rc = check_kind(c, realkind)) return rc;
     if (!c->avg.p) return fail(c, LBM_ESTATE, "no averages: call lbm_set_averaging first");
     if (int rc = average_flush(c)) return rc;
-    const Layout& L = c->lay;
-    const int rb = c->ops->real_bytes;
-    const size_t P = (size_t)L.cplane;
-    std::vector<unsigned char> img(6 * P * rb);
-    HIPCHK(c, hipMemcpyAsync(img.data(), c->avg.p, img.size(), hipMemcpyDeviceToHost, c->stream));
-    HIPCHK(c, hipStreamSynchronize(c->stream));
-    if (count) *count = c->avg_count;
-    const size_t nc = ncell_padded(c);
+    const size_t cb = ncell_padded(c) * realkind;
     void* out[4] = {uave, vave, wave, ti};
-    for (int q = 0; q < 4; ++q)
-        if (out[q]) std::memset(out[q], 0, nc * realkind);
-    if (c->avg_count == 0) return LBM_OK;
-    auto put = [&](void* o, size_t idx, double v) {
-        if (!o) return;
-        if (realkind == 8) static_cast<double*>(o)[idx] = v;
-        else static_cast<float*>(o)[idx] = (float)v;
-    };
-    const bool f32 = rb == 4;
-    for (int k = 1; k <= L.nz; ++k)
-        for (int j = 1; j <= L.ny; ++j)
-            for (int i = 1; i <= L.nx; ++i) {
-                const size_t o = (size_t)L.cidx(i, j, k);
-                const size_t hc = ((size_t)k * (L.ny + 2) + j) * (L.nx + 2) + i;
-                double m[3], m2[3];
-                for (int q = 0; q < 3; ++q) {
-                    m[q] = get_real(img.data(), q * P + o, rb) / c->avg_count;
-                    m2[q] = get_real(img.data(), (3 + q) * P + o, rb) / c->avg_count;
-                    if (f32) {
-                        m[q] = (float)m[q];
-                        m2[q] = (float)m2[q];
-                    }
-                }
-                // src/m_averaging_full_kernelfin.F90:46-60
-                double t = 0.0;
-                for (int q = 0; q < 3; ++q) {
-                    const double var = f32 ? (double)((float)m2[q] - (float)m[q] * (float)m[q]) : m2[q] - m[q] * m[q];
-                    t += var > 0.0 ? var : 0.0;
-                }
-                t = f32 ? (double)((float)t / 3.0f) : t / 3.0;
-                put(uave, hc, m[0]);
-                put(vave, hc, m[1]);
-                put(wave, hc, m[2]);
-                put(ti, hc, f32 ? (double)std::sqrt((float)(t > 0.0 ? t : 0.0)) : std::sqrt(t > 0.0 ? t : 0.0));
-            }
+    if (c->avg_count == 0) {
+        HIPCHK(c, hipStreamSynchronize(c->stream));
+        for (void* o : out)
+            if (o) std::memset(o, 0, cb);
+    } else {
+        if (int rc = dev_alloc(c, c->stage, 4 * cb)) return rc;
+        char* st = static_cast<char*>(c->stage.p);
+        HIPCHK(c, c->ops->averages_out(c->lay, c->avg.p, c->avg_count, st, realkind, c->stream));
+        for (int q = 0; q < 4; ++q)
+            if (out[q]) HIPCHK(c, hipMemcpyAsync(out[q], st + q * cb, cb, hipMemcpyDeviceToHost, c->stream));
+        HIPCHK(c, hipStreamSynchronize(c->stream));
+    }
+    if (count) *count = c->avg_count;
     return LBM_OK;
 }
 
@@ -850,7 +821,7 @@ int lbm_get_state(lbm_ctx* c, void* f, int realkind) {
     const void* cur = c->buf[c->cur];
     const int g = c->pending ? c->cur : c->cur ^ 1;
     HIPCHK(c, c->ops->state_out(c->lay, cur, c->buf[g], c->pending ? 0 : 1, c->ghost_raw[g] ? 1 : 0, c->stage.p,
-                                nullptr, nullptr, nullptr, nullptr, realkind, c->stream));
+                                realkind, c->stream));
     HIPCHK(c, hipMemcpyAsync(f, c->stage.p, n * realkind, hipMemcpyDeviceToHost, c->stream));
     HIPCHK(c, hipStreamSynchronize(c->stream));
     return LBM_OK;
@@ -864,17 +835,24 @@ int lbm_get_macros(lbm_ctx* c, void* rho, void* u, void* v, void* w, int realkin
     if (int rc = check_kind(c, realkind)) return rc;
     const size_t nc = ncell_padded(c);
     const size_t cb = nc * realkind;
-    if (int rc = dev_alloc(c, c->stage, 4 * cb)) return rc;
+    // the four fields and the kernel's instability flag
+    if (int rc = dev_alloc(c, c->stage, 4 * cb + sizeof(int))) return rc;
     char* st = static_cast<char*>(c->stage.p);
+    int* flag = reinterpret_cast<int*>(st + 4 * cb);
     const int g = c->pending ? c->cur : c->cur ^ 1;
-    HIPCHK(c, c->ops->state_out(c->lay, c->buf[c->cur], c->buf[g], c->pending ? 0 : 1, c->ghost_raw[g] ? 1 : 0,
-                                nullptr, st, st + cb, st + 2 * cb, st + 3 * cb, realkind, c->stream));
+    HIPCHK(c, hipMemsetAsync(flag, 0, sizeof(int), c->stream));
+    HIPCHK(c, c->ops->moments_out(c->lay, c->buf[c->cur], c->buf[g], c->pending ? 0 : 1, c->ghost_raw[g] ? 1 : 0, st,
+                                  flag, realkind, c->stream));
     HIPCHK(c, hipMemcpyAsync(rho, st, cb, hipMemcpyDeviceToHost, c->stream));
     HIPCHK(c, hipMemcpyAsync(u, st + cb, cb, hipMemcpyDeviceToHost, c->stream));
     HIPCHK(c, hipMemcpyAsync(v, st + 2 * cb, cb, hipMemcpyDeviceToHost, c->stream));
     HIPCHK(c, hipMemcpyAsync(w, st + 3 * cb, cb, hipMemcpyDeviceToHost, c->stream));
+    int unstable = 0;
+    HIPCHK(c, hipMemcpyAsync(&unstable, flag, sizeof(int), hipMemcpyDeviceToHost, c->stream));
     HIPCHK(c, hipStreamSynchronize(c->stream));
-    // the instability test of src/m_diag.F90:169-173 on the moments just returned (all cells)
+    if (!unstable) return LBM_OK;
+    // the instability test of src/m_diag.F90:169-173 on the moments just returned (all cells): what
+    // the flag stands for, counted for the message
     size_t bad = 0, nonpos = 0;
     double rmin = INFINITY;
     const void* arr[4] = {rho, u, v, w};
@@ -1064,6 +1042,24 @@ int lbm_generate_turbulence(lbm_ctx* c, int nrturb, double ampl, uint64_t seed, 
     return LBM_OK;
 }
 
+namespace {
+// nv reals per cell in the reference's layout -> nv per-cell arrays of the compute type, turned on
+// the device (fields.h)
+int upload_field(lbm_ctx* c, int nv, const void* host, int realkind, DevBuf* to) {
+    const size_t n = (size_t)nv * ncell_padded(c) * realkind;
+    void* p[3] = {nullptr, nullptr, nullptr};
+    if (int rc = dev_alloc(c, c->stage, n)) return rc;
+    for (int q = 0; q < nv; ++q) {
+        if (int rc = dev_alloc(c, to[q], (size_t)c->lay.cplane * c->ops->real_bytes)) return rc;
+        p[q] = to[q].p;
+    }
+    HIPCHK(c, hipMemcpyAsync(c->stage.p, host, n, hipMemcpyHostToDevice, c->stream));
+    HIPCHK(c, c->ops->field_in(c->lay, nv, c->stage.p, realkind, p, c->stream));
+    HIPCHK(c, hipStreamSynchronize(c->stream));
+    return LBM_OK;
+}
+}  // namespace
+
 int lbm_set_external_forcing(lbm_ctx* c, const void* force, int realkind) {
     if (int rc_ = check_ctx(c)) return rc_;
     if (int rc = check_no_part(c)) return rc;
@@ -1073,24 +1069,7 @@ int lbm_set_external_forcing(lbm_ctx* c, const void* force, int realkind) {
         return LBM_OK;
     }
     if (int rc = check_kind(c, realkind)) return rc;
-    const Layout& L = c->lay;
-    const size_t nc = ncell_padded(c);
-    const int rb = c->ops->real_bytes;
-    for (int q = 0; q < 3; ++q) {
-        std::vector<unsigned char> plane((size_t)L.cplane * rb, 0);
-        for (int k = 0; k <= L.nz + 1; ++k)
-            for (int j = 0; j <= L.ny + 1; ++j)
-                for (int i = 0; i <= L.nx + 1; ++i) {
-                    const size_t hc = ((size_t)k * (L.ny + 2) + j) * (L.nx + 2) + i;
-                    const double v = realkind == 8 ? static_cast<const double*>(force)[3 * hc + q]
-                                                   : static_cast<const float*>(force)[3 * hc + q];
-                    put_real(plane.data(), (size_t)L.cidx(i, j, k), v, rb);
-                }
-        if (int rc = dev_alloc(c, c->force[q], plane.size())) return rc;
-        HIPCHK(c, hipMemcpyAsync(c->force[q].p, plane.data(), plane.size(), hipMemcpyHostToDevice, c->stream));
-        HIPCHK(c, hipStreamSynchronize(c->stream));
-    }
-    (void)nc;
+    if (int rc = upload_field(c, 3, force, realkind, c->force)) return rc;
     c->has_force = true;
     return LBM_OK;
 }
@@ -1105,21 +1084,7 @@ int lbm_set_buoyancy(lbm_ctx* c, const void* pottemp, double theta0, double scal
     if (int rc = check_kind(c, realkind)) return rc;
     if (!(theta0 != 0.0) || !std::isfinite(theta0) || !std::isfinite(scaling))
         return fail(c, LBM_EINVAL, "buoyancy: theta0 must be finite and non-zero, scaling finite");
-    // the reference layout (0:nx+1, 0:ny+1, 0:nz+1) -> the cell layout of the compute type
-    const Layout& L = c->lay;
-    const int rb = c->ops->real_bytes;
-    std::vector<unsigned char> img((size_t)L.cplane * rb, 0);
-    for (int k = 0; k <= L.nz + 1; ++k)
-        for (int j = 0; j <= L.ny + 1; ++j)
-            for (int i = 0; i <= L.nx + 1; ++i) {
-                const size_t hc = ((size_t)k * (L.ny + 2) + j) * (L.nx + 2) + i;
-                const double v = realkind == 8 ? static_cast<const double*>(pottemp)[hc]
-                                               : static_cast<const float*>(pottemp)[hc];
-                put_real(img.data(), (size_t)L.cidx(i, j, k), v, rb);
-            }
-    if (int rc = dev_alloc(c, c->theta, img.size())) return rc;
-    HIPCHK(c, hipMemcpyAsync(c->theta.p, img.data(), img.size(), hipMemcpyHostToDevice, c->stream));
-    HIPCHK(c, hipStreamSynchronize(c->stream));
+    if (int rc = upload_field(c, 1, pottemp, realkind, &c->theta)) return rc;
     c->btheta0 = round_real(c, theta0);
     c->bscale = round_real(c, scaling);
     c->buoy_on = true;

@@ -103,6 +103,8 @@ int finish_totals(lbm_ctx* c, const double* partial, int nb, double* mass, doubl
 int check_no_part(lbm_ctx* c);
 int hipfail(lbm_ctx* c, hipError_t e, const char* where);
 int dev_alloc(lbm_ctx* c, DevBuf& b, size_t n);
+// cells of the padded grid
+size_t ncell_padded(const lbm_ctx* c);
 void dev_free(DevBuf& b);
 double round_real(const lbm_ctx* c, double v);
 // element q of a host image of a device array of the compute type (rb bytes per value)

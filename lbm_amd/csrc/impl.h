@@ -136,9 +136,17 @@ struct Ops {
                          double rho0, hipStream_t);
     hipError_t (*aos_in)(const Layout&, const void* aos, int realkind, void* dstA, void* dstB, hipStream_t);
     hipError_t (*state_out)(const Layout&, const void* cur, const void* gsrc, int stream_interior, int ghost_raw,
-                            void* aos, void* rho, void* u, void* v, void* w, int realkind, hipStream_t);
-    hipError_t (*feq_init)(const Layout&, int bgk3, const void* rho, const void* u, const void* v, const void* w,
-                           int realkind, void* dst, void* mr, void* mu, void* mv, void* mw, hipStream_t);
+                            void* aos, int realkind, hipStream_t);
+    // rho, u, v, w one after the other; *unstable (device) is set, never cleared
+    hipError_t (*moments_out)(const Layout&, const void* cur, const void* gsrc, int stream_interior, int ghost_raw,
+                              void* out, int* unstable, int realkind, hipStream_t);
+    // uave, vave, wave, ti one after the other from the six sums of count steps
+    hipError_t (*averages_out)(const Layout&, const void* avg, int count, void* out, int realkind, hipStream_t);
+    // nv = 1 or 3 reals per cell in the reference's order into nv per-cell arrays of the compute type
+    hipError_t (*field_in)(const Layout&, int nv, const void* in, int realkind, void* const* to, hipStream_t);
+    // moments rho, u, v, w one after the other; m: their per-cell arrays
+    hipError_t (*feq_init)(const Layout&, int bgk3, const void* moments, int realkind, void* dst, void* const* m,
+                           hipStream_t);
     hipError_t (*totals)(const Layout&, const void* cur, int stream_interior, double* partial, int nblocks,
                          hipStream_t);
     hipError_t (*average)(const Layout&, const void* cur, int stream_interior, void* avg, hipStream_t);

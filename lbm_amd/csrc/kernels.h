@@ -9,7 +9,7 @@
 //                         corners; inflow/outflow).
 // The buffers hold post-collision populations (the reference's f1 after postcoll/solids) in
 // the interior and the reference's persistent ghost layers.  The reference's post-streaming
-// state f1 = drift(P(n)) is formed on the fly by the next step, and by state_out_kernel when the
+// state f1 = drift(P(n)) is formed on the fly by the next step, and by StateOut when the
 // caller asks for it.
 #pragma once
 
@@ -20,6 +20,7 @@
 #include <type_traits>
 
 #include "codec.h"
+#include "fields.h"
 #include "lattice.h"
 #include "layout.h"
 #include "impl.h"
@@ -1180,95 +1181,108 @@ __global__ void clock_tick_kernel(int* clock) {
 }
 
 // ------------------------------------------------------------------------------------------
-// State transfer between the reference's AoS layout f(nl,0:nx+1,0:ny+1,0:nz+1) (H = float or
-// double, as the caller's REAL kind) and the device buffers.
+// State transfer between the reference's layout f(nl,0:nx+1,0:ny+1,0:nz+1) and the device buffers
+// (H = float or double, the caller's REAL kind): what the tiled kernels of fields.h do with a cell.
 // ------------------------------------------------------------------------------------------
-template <int Q, class C, typename H>
-__global__ void aos_to_soa_kernel(Layout L, const H* __restrict__ aos, void* dstA, void* dstB) {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    const int j = blockIdx.y;
-    const int k = blockIdx.z;
-    if (i > L.nx + 1) return;
-    const size_t base = ((size_t)k * (L.ny + 2) * (L.nx + 2) + (size_t)j * (L.nx + 2) + i) * Q;
-    const int oc = L.cell(i, j, k);
+template <int Q, class C>
+struct StateIn {
+    void* a;
+    void* b;   // nullptr: one buffer only
+    template <typename H>
+    __device__ void operator()(const Layout& L, int i, int j, int k, const H (&f)[Q]) const {
+        const int oc = L.cell(i, j, k);
 #pragma unroll
-    for (int l = 0; l < Q; ++l) {
-        const typename C::real v = (typename C::real)aos[base + l];
-        st<Q, C>(L, dstA, l, oc, v);
-        if (dstB) st<Q, C>(L, dstB, l, oc, v);
+        for (int l = 0; l < Q; ++l) {
+            const typename C::real v = (typename C::real)f[l];
+            st<Q, C>(L, a, l, oc, v);
+            if (b) st<Q, C>(L, b, l, oc, v);
+        }
     }
-}
+};
 
-// The reference's f1 (post-streaming state including ghosts) and/or its moments
-// (src/m_macrovars_kernel.F90:41-49, all cells including ghosts).
+// The reference's f1 (post-streaming state including ghosts):
 //   interior: stream_interior ? cur(l, x - c) : cur(l, x)
 //   ghosts  : ghost_raw ? gsrc(l, x) as stored : gsrc(l, x with periodic axes wrapped)
-template <int Q, class C, typename H>
-__global__ void state_out_kernel(Layout L, const void* cur, const void* gsrc, int stream_interior, int ghost_raw,
-                                 H* __restrict__ aos, H* rho, H* u, H* v, H* w) {
-    using R = typename C::real;
-    using Lt = Lattice<Q>;
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    const int j = blockIdx.y;
-    const int k = blockIdx.z;
-    if (i > L.nx + 1) return;
-    const bool interior = i >= 1 && i <= L.nx && j >= 1 && j <= L.ny && k >= 1 && k <= L.nz;
-    const size_t cidx = (size_t)k * (L.ny + 2) * (L.nx + 2) + (size_t)j * (L.nx + 2) + i;
-    R tr = 0, tu = 0, tv = 0, tw = 0;
+template <int Q, class C>
+struct StateOut {
+    const void* cur;
+    const void* gsrc;
+    int stream_interior, ghost_raw;
+    __device__ void cell(const Layout& L, int i, int j, int k, typename C::real (&f)[Q]) const {
+        using Lt = Lattice<Q>;
+        const bool interior = interior_cell(L, i, j, k);
 #pragma unroll
-    for (int l = 0; l < Q; ++l) {
-        R f;
-        if (interior) {
-            const int s = stream_interior;
-            f = ld<Q, C>(L, cur, l, L.cell_w(i - s * Lt::cx(l), j - s * Lt::cy(l), k - s * Lt::cz(l)));
-        } else {
-            f = ld<Q, C>(L, gsrc, l, ghost_raw ? L.cell(i, j, k) : L.cell_w(i, j, k));
+        for (int l = 0; l < Q; ++l) {
+            if (interior) {
+                const int s = stream_interior;
+                f[l] = ld<Q, C>(L, cur, l, L.cell_w(i - s * Lt::cx(l), j - s * Lt::cy(l), k - s * Lt::cz(l)));
+            } else {
+                f[l] = ld<Q, C>(L, gsrc, l, ghost_raw ? L.cell(i, j, k) : L.cell_w(i, j, k));
+            }
         }
-        if (aos) aos[cidx * Q + l] = (H)f;
-        tr += f;
-        if (Lt::cx(l) > 0) tu += f; else if (Lt::cx(l) < 0) tu -= f;
-        if (Lt::cy(l) > 0) tv += f; else if (Lt::cy(l) < 0) tv -= f;
-        if (Lt::cz(l) > 0) tw += f; else if (Lt::cz(l) < 0) tw -= f;
     }
-    if (rho) {
+    template <typename H>
+    __device__ void operator()(const Layout& L, int i, int j, int k, H (&o)[Q]) const {
+        typename C::real f[Q];
+        cell(L, i, j, k, f);
+#pragma unroll
+        for (int l = 0; l < Q; ++l) o[l] = (H)f[l];
+    }
+};
+
+// Its moments rho, u, v, w (src/m_macrovars_kernel.F90:41-49, all cells including ghosts).  *unstable
+// becomes non-zero if one of them is not finite or a density is not positive
+// (src/m_diag.F90:169-173): every cell that sees it writes the same value.
+template <int Q, class C>
+struct MomentsOut {
+    StateOut<Q, C> state;
+    int* unstable;
+    template <typename H>
+    __device__ void operator()(const Layout& L, int i, int j, int k, H (&o)[4]) const {
+        using R = typename C::real;
+        using Lt = Lattice<Q>;
+        R f[Q];
+        state.cell(L, i, j, k, f);
+        R tr = 0, tu = 0, tv = 0, tw = 0;
+#pragma unroll
+        for (int l = 0; l < Q; ++l) {
+            tr += f[l];
+            if (Lt::cx(l) > 0) tu += f[l]; else if (Lt::cx(l) < 0) tu -= f[l];
+            if (Lt::cy(l) > 0) tv += f[l]; else if (Lt::cy(l) < 0) tv -= f[l];
+            if (Lt::cz(l) > 0) tw += f[l]; else if (Lt::cz(l) < 0) tw -= f[l];
+        }
         const R inv = R(1) / tr;
-        rho[cidx] = (H)tr;
-        u[cidx] = (H)(tu * inv);
-        v[cidx] = (H)(tv * inv);
-        w[cidx] = (H)(tw * inv);
+        o[0] = (H)tr;
+        o[1] = (H)(tu * inv);
+        o[2] = (H)(tv * inv);
+        o[3] = (H)(tw * inv);
+        if (!(isfinite(o[0]) && isfinite(o[1]) && isfinite(o[2]) && isfinite(o[3]) && o[0] > H(0))) *unstable = 1;
     }
-}
+};
 
 // Equilibrium initialisation (src/m_fequil3_kernel.F90 then src/m_fillghosts.F90): every cell,
-// ghosts included, gets feq of its clamped interior cell.  The moments (H, reference cell
-// layout) are also kept in the device cell layout for the first collision.
-template <int Q, class C, bool BGK3, typename H>
-__global__ void feq_init_kernel(Layout L, const H* rho, const H* u, const H* v, const H* w, void* dst,
-                                typename C::real* mr, typename C::real* mu, typename C::real* mv,
-                                typename C::real* mw) {
-    using R = typename C::real;
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    const int j = blockIdx.y;
-    const int k = blockIdx.z;
-    if (i > L.nx + 1) return;
-    const int i1 = i < 1 ? 1 : (i > L.nx ? L.nx : i);
-    const int j1 = j < 1 ? 1 : (j > L.ny ? L.ny : j);
-    const int k1 = k < 1 ? 1 : (k > L.nz ? L.nz : k);
-    const size_t c = (size_t)k1 * (L.ny + 2) * (L.nx + 2) + (size_t)j1 * (L.nx + 2) + i1;
-    const R r = (R)rho[c], ux = (R)u[c], uy = (R)v[c], uz = (R)w[c];
-    const R usq = ux * ux + uy * uy + uz * uz;
-    const int oc = L.cell(i, j, k);
+// ghosts included, gets feq of its clamped interior cell, whose moments v holds.  The moments are
+// also kept in the device cell layout for the first collision.
+template <int Q, class C, bool BGK3>
+struct EquilibriumIn {
+    void* dst;
+    typename C::real *mr, *mu, *mv, *mw;
+    template <typename H>
+    __device__ void operator()(const Layout& L, int i, int j, int k, const H (&v)[4]) const {
+        using R = typename C::real;
+        const R r = (R)v[0], ux = (R)v[1], uy = (R)v[2], uz = (R)v[3];
+        const R usq = ux * ux + uy * uy + uz * uz;
+        const int oc = L.cell(i, j, k);
 #pragma unroll
-    for (int l = 0; l < Q; ++l)
-        st<Q, C>(L, dst, l, oc, feq_dir<Q, BGK3, R>(l, r, ux, uy, uz, usq));
-    if (i == i1 && j == j1 && k == k1) {
-        const int ox = L.cidx(i, j, k);
-        mr[ox] = r; mu[ox] = ux; mv[ox] = uy; mw[ox] = uz;
+        for (int l = 0; l < Q; ++l)
+            st<Q, C>(L, dst, l, oc, feq_dir<Q, BGK3, R>(l, r, ux, uy, uz, usq));
+        if (interior_cell(L, i, j, k)) {
+            const int ox = L.cidx(i, j, k);
+            mr[ox] = r; mu[ox] = ux; mv[ox] = uy; mw[ox] = uz;
+        }
     }
-}
+};
 
-// Global mass and momentum of the state (interior cells) in FP64: per-block partial sums,
-// finished on the host.  partial[4*block + {0,1,2,3}] = (mass, mx, my, mz).
 // Adds the moments of the current state (streamed when stream_interior) to the averaging sums.
 template <int Q, class C>
 __global__ void average_kernel(Layout L, const void* cur, int stream_interior, typename C::real* avg) {

@@ -31,8 +31,6 @@ struct Limits<Dual> {
     static Dual eps() { return Dual(std::sqrt(DBL_MIN)); }
 };
 
-inline dim3 grid_cells(const Layout& L, int bx) { return dim3((L.nx + 2 + bx - 1) / bx, L.ny + 2, L.nz + 2); }
-
 template <int Q, class C>
 struct Launch {
     using R = typename C::real;
@@ -273,49 +271,52 @@ struct Launch {
     }
 
     static hipError_t aos_in(const Layout& L, const void* aos, int realkind, void* dA, void* dB, hipStream_t s) {
-        const dim3 block(128, 1, 1);
-        const dim3 grid = grid_cells(L, 128);
-        if (realkind == 8)
-            hipLaunchKernelGGL((aos_to_soa_kernel<Q, C, double>), grid, block, 0, s, L, static_cast<const double*>(aos), dA, dB);
-        else
-            hipLaunchKernelGGL((aos_to_soa_kernel<Q, C, float>), grid, block, 0, s, L, static_cast<const float*>(aos), dA, dB);
-        return hipGetLastError();
+        const StateIn<Q, C> f{dA, dB};
+        if (realkind == 8) return cells_in<Q, true, false>(L, f, static_cast<const double*>(aos), s);
+        return cells_in<Q, true, false>(L, f, static_cast<const float*>(aos), s);
     }
 
-    static hipError_t state_out(const Layout& L, const void* cur, const void* gsrc, int si, int raw, void* aos,
-                                void* rho, void* u, void* v, void* w, int realkind, hipStream_t s) {
-        const dim3 block(128, 1, 1);
-        const dim3 grid = grid_cells(L, 128);
-        if (realkind == 8)
-            hipLaunchKernelGGL((state_out_kernel<Q, C, double>), grid, block, 0, s, L, cur, gsrc, si, raw,
-                               static_cast<double*>(aos), static_cast<double*>(rho), static_cast<double*>(u),
-                               static_cast<double*>(v), static_cast<double*>(w));
-        else
-            hipLaunchKernelGGL((state_out_kernel<Q, C, float>), grid, block, 0, s, L, cur, gsrc, si, raw,
-                               static_cast<float*>(aos), static_cast<float*>(rho), static_cast<float*>(u),
-                               static_cast<float*>(v), static_cast<float*>(w));
-        return hipGetLastError();
+    static hipError_t state_out(const Layout& L, const void* cur, const void* gsrc, int si, int raw, void* aos, int realkind,
+                                hipStream_t s) {
+        const StateOut<Q, C> f{cur, gsrc, si, raw};
+        if (realkind == 8) return cells_out<Q, true>(L, f, static_cast<double*>(aos), s);
+        return cells_out<Q, true>(L, f, static_cast<float*>(aos), s);
     }
 
-    template <typename H>
-    static hipError_t feq_init_h(const Layout& L, int bgk3, const void* r, const void* u, const void* v, const void* w,
-                                 void* dst, void* mr, void* mu, void* mv, void* mw, hipStream_t s) {
-        const dim3 block(128, 1, 1);
-        const dim3 grid = grid_cells(L, 128);
-        const H *hr = static_cast<const H*>(r), *hu = static_cast<const H*>(u), *hv = static_cast<const H*>(v),
-                *hw = static_cast<const H*>(w);
-        R *pr = static_cast<R*>(mr), *pu = static_cast<R*>(mu), *pv = static_cast<R*>(mv), *pw = static_cast<R*>(mw);
-        if (bgk3)
-            hipLaunchKernelGGL((feq_init_kernel<Q, C, true, H>), grid, block, 0, s, L, hr, hu, hv, hw, dst, pr, pu, pv, pw);
-        else
-            hipLaunchKernelGGL((feq_init_kernel<Q, C, false, H>), grid, block, 0, s, L, hr, hu, hv, hw, dst, pr, pu, pv, pw);
-        return hipGetLastError();
+    static hipError_t moments_out(const Layout& L, const void* cur, const void* gsrc, int si, int raw, void* out,
+                                  int* unstable, int realkind, hipStream_t s) {
+        const MomentsOut<Q, C> f{{cur, gsrc, si, raw}, unstable};
+        if (realkind == 8) return cells_out<4, false>(L, f, static_cast<double*>(out), s);
+        return cells_out<4, false>(L, f, static_cast<float*>(out), s);
     }
 
-    static hipError_t feq_init(const Layout& L, int bgk3, const void* r, const void* u, const void* v, const void* w,
-                               int realkind, void* dst, void* mr, void* mu, void* mv, void* mw, hipStream_t s) {
-        if (realkind == 8) return feq_init_h<double>(L, bgk3, r, u, v, w, dst, mr, mu, mv, mw, s);
-        return feq_init_h<float>(L, bgk3, r, u, v, w, dst, mr, mu, mv, mw, s);
+    static hipError_t averages_out(const Layout& L, const void* avg, int count, void* out, int realkind, hipStream_t s) {
+        const AveragesOut<R> f{static_cast<const R*>(avg), (double)count};
+        if (realkind == 8) return cells_out<4, false>(L, f, static_cast<double*>(out), s);
+        return cells_out<4, false>(L, f, static_cast<float*>(out), s);
+    }
+
+    template <int NV>
+    static hipError_t field_in_n(const Layout& L, const void* in, int realkind, void* const* to, hipStream_t s) {
+        CellsIn<NV, R> f;
+        for (int q = 0; q < NV; ++q) f.to[q] = static_cast<R*>(to[q]);
+        if (realkind == 8) return cells_in<NV, true, false>(L, f, static_cast<const double*>(in), s);
+        return cells_in<NV, true, false>(L, f, static_cast<const float*>(in), s);
+    }
+    static hipError_t field_in(const Layout& L, int nv, const void* in, int realkind, void* const* to, hipStream_t s) {
+        return nv == 3 ? field_in_n<3>(L, in, realkind, to, s) : field_in_n<1>(L, in, realkind, to, s);
+    }
+
+    template <bool B3>
+    static hipError_t feq_init_t(const Layout& L, const void* in, int realkind, void* dst, void* const* m, hipStream_t s) {
+        const EquilibriumIn<Q, C, B3> f{dst, static_cast<R*>(m[0]), static_cast<R*>(m[1]), static_cast<R*>(m[2]),
+                                        static_cast<R*>(m[3])};
+        if (realkind == 8) return cells_in<4, false, true>(L, f, static_cast<const double*>(in), s);
+        return cells_in<4, false, true>(L, f, static_cast<const float*>(in), s);
+    }
+    static hipError_t feq_init(const Layout& L, int bgk3, const void* in, int realkind, void* dst, void* const* m,
+                               hipStream_t s) {
+        return bgk3 ? feq_init_t<true>(L, in, realkind, dst, m, s) : feq_init_t<false>(L, in, realkind, dst, m, s);
     }
 
     static hipError_t totals(const Layout& L, const void* cur, int si, double* partial, int nblocks, hipStream_t s) {
@@ -446,7 +447,8 @@ struct Launch {
     }
 
     static const Ops* ops() {
-        static const Ops o = {&step, &closed, &snapshot, &edges, &inflow, &aos_in, &state_out, &feq_init, &totals, &average,
+        static const Ops o = {&step, &closed, &snapshot, &edges, &inflow, &aos_in, &state_out, &moments_out,
+                              &averages_out, &field_in, &feq_init, &totals, &average,
                               sizeof(MemberTab<R>), &ens_pack, &ens_step,
                               kAdj ? &adj_step : nullptr, kAdj ? &adj_inflow : nullptr, kAdj ? &adj_face : nullptr,
                               &objective, &halo_pack, &halo_unpack, &ghost_copy, &turb_step, (int)sizeof(R),
