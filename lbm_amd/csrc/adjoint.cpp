@@ -19,6 +19,7 @@
 #include "fields.h"
 #include "impl.h"
 #include "layout.h"
+#include "transfer.h"
 
 using namespace lbm;
 using namespace lbm_host;
@@ -253,7 +254,8 @@ int lbm_adjoint_run(lbm_ctx* c, int it0, int nsteps, int every, const int32_t* b
             // the gradient in the reference's layout
             if (int r = dev_alloc(c, c->stage, gbytes)) return r;
             HIPCHK(c, (cells_out<3, true>(c->lay, GradientOut{gFp}, static_cast<double*>(c->stage.p), c->stream)));
-            HIPCHK(c, hipMemcpyAsync(grad_force, c->stage.p, gbytes, hipMemcpyDeviceToHost, c->stream));
+            const HostPart part{grad_force, 0, gbytes};
+            if (int r = copy_out(c, c->stage.p, &part, 1)) return r;
         }
         HIPCHK(c, hipMemcpyAsync(ha.data(), acc.p, ha.size() * sizeof(double), hipMemcpyDeviceToHost, c->stream));
         HIPCHK(c, hipMemcpyAsync(hs.data(), gS.p, hs.size() * sizeof(double), hipMemcpyDeviceToHost, c->stream));

@@ -17,6 +17,7 @@
 #include "impl.h"
 #include "layout.h"
 #include "dual.h"
+#include "transfer.h"
 
 using namespace lbm;
 using namespace lbm_host;
@@ -474,6 +475,7 @@ int lbm_create(const lbm_desc* desc, lbm_ctx** out) {
     if (e != hipSuccess || ndev == 0) return fail(nullptr, LBM_EHIP, std::string("no HIP device: ") + hipGetErrorString(e));
 
     lbm_ctx* c = new lbm_ctx();
+    transfer_retain();
     c->d = d;
     c->d.block_x = bx;
     c->d.block_y = by;
@@ -577,6 +579,7 @@ int lbm_destroy(lbm_ctx* c) {
     for (hipEvent_t ev : c->ev_step) hipEventDestroy(ev);
     for (hipEvent_t ev : c->ev_bc) hipEventDestroy(ev);
     if (c->stream) hipStreamDestroy(c->stream);
+    transfer_release();
     delete c;
     return LBM_OK;
 }
@@ -588,7 +591,8 @@ int lbm_set_state(lbm_ctx* c, const void* f, int realkind) {
     if (int rc = check_kind(c, realkind)) return rc;
     const size_t n = ncell_padded(c) * c->d.q;
     if (int rc = dev_alloc(c, c->stage, n * realkind)) return rc;
-    HIPCHK(c, hipMemcpyAsync(c->stage.p, f, n * realkind, hipMemcpyHostToDevice, c->stream));
+    const HostPart part{const_cast<void*>(f), 0, n * realkind};
+    if (int rc = copy_in(c, c->stage.p, &part, 1)) return rc;
     HIPCHK(c, c->ops->aos_in(c->lay, c->stage.p, realkind, c->buf[0], c->buf[1], c->stream));
     HIPCHK(c, hipStreamSynchronize(c->stream));
     c->cur = 0;
@@ -614,10 +618,10 @@ int lbm_init_equilibrium(lbm_ctx* c, const void* rho, const void* u, const void*
     for (int q = 0; q < 4; ++q)
         if (int rc = dev_alloc(c, c->ext[q], mb)) return rc;
     char* st = static_cast<char*>(c->stage.p);
-    HIPCHK(c, hipMemcpyAsync(st, rho, cb, hipMemcpyHostToDevice, c->stream));
-    HIPCHK(c, hipMemcpyAsync(st + cb, u, cb, hipMemcpyHostToDevice, c->stream));
-    HIPCHK(c, hipMemcpyAsync(st + 2 * cb, v, cb, hipMemcpyHostToDevice, c->stream));
-    HIPCHK(c, hipMemcpyAsync(st + 3 * cb, w, cb, hipMemcpyHostToDevice, c->stream));
+    const void* host[4] = {rho, u, v, w};
+    HostPart parts[4];
+    for (size_t q = 0; q < 4; ++q) parts[q] = {const_cast<void*>(host[q]), q * cb, cb};
+    if (int rc = copy_in(c, st, parts, 4)) return rc;
     // fB = feq with clamped ghosts; fA = fB; boundarycond(fB,fA); boundarycond(fA,fB)
     void* const ext[4] = {c->ext[0].p, c->ext[1].p, c->ext[2].p, c->ext[3].p};
     HIPCHK(c, c->ops->feq_init(c->lay, c->d.ibgk == 3, st, realkind, c->buf[1], ext, c->stream));
@@ -802,9 +806,9 @@ int lbm_get_averages(lbm_ctx* c, void* uave, void* vave, void* wave, void* ti, i
         if (int rc = dev_alloc(c, c->stage, 4 * cb)) return rc;
         char* st = static_cast<char*>(c->stage.p);
         HIPCHK(c, c->ops->averages_out(c->lay, c->avg.p, c->avg_count, st, realkind, c->stream));
-        for (int q = 0; q < 4; ++q)
-            if (out[q]) HIPCHK(c, hipMemcpyAsync(out[q], st + q * cb, cb, hipMemcpyDeviceToHost, c->stream));
-        HIPCHK(c, hipStreamSynchronize(c->stream));
+        HostPart parts[4];
+        for (size_t q = 0; q < 4; ++q) parts[q] = {out[q], q * cb, cb};
+        if (int rc = copy_out(c, st, parts, 4)) return rc;
     }
     if (count) *count = c->avg_count;
     return LBM_OK;
@@ -822,9 +826,8 @@ int lbm_get_state(lbm_ctx* c, void* f, int realkind) {
     const int g = c->pending ? c->cur : c->cur ^ 1;
     HIPCHK(c, c->ops->state_out(c->lay, cur, c->buf[g], c->pending ? 0 : 1, c->ghost_raw[g] ? 1 : 0, c->stage.p,
                                 realkind, c->stream));
-    HIPCHK(c, hipMemcpyAsync(f, c->stage.p, n * realkind, hipMemcpyDeviceToHost, c->stream));
-    HIPCHK(c, hipStreamSynchronize(c->stream));
-    return LBM_OK;
+    const HostPart part{f, 0, n * realkind};
+    return copy_out(c, c->stage.p, &part, 1);
 }
 
 int lbm_get_macros(lbm_ctx* c, void* rho, void* u, void* v, void* w, int realkind) {
@@ -843,13 +846,9 @@ int lbm_get_macros(lbm_ctx* c, void* rho, void* u, void* v, void* w, int realkin
     HIPCHK(c, hipMemsetAsync(flag, 0, sizeof(int), c->stream));
     HIPCHK(c, c->ops->moments_out(c->lay, c->buf[c->cur], c->buf[g], c->pending ? 0 : 1, c->ghost_raw[g] ? 1 : 0, st,
                                   flag, realkind, c->stream));
-    HIPCHK(c, hipMemcpyAsync(rho, st, cb, hipMemcpyDeviceToHost, c->stream));
-    HIPCHK(c, hipMemcpyAsync(u, st + cb, cb, hipMemcpyDeviceToHost, c->stream));
-    HIPCHK(c, hipMemcpyAsync(v, st + 2 * cb, cb, hipMemcpyDeviceToHost, c->stream));
-    HIPCHK(c, hipMemcpyAsync(w, st + 3 * cb, cb, hipMemcpyDeviceToHost, c->stream));
     int unstable = 0;
-    HIPCHK(c, hipMemcpyAsync(&unstable, flag, sizeof(int), hipMemcpyDeviceToHost, c->stream));
-    HIPCHK(c, hipStreamSynchronize(c->stream));
+    const HostPart parts[5] = {{rho, 0, cb}, {u, cb, cb}, {v, 2 * cb, cb}, {w, 3 * cb, cb}, {&unstable, 4 * cb, sizeof(int)}};
+    if (int rc = copy_out(c, st, parts, 5)) return rc;
     if (!unstable) return LBM_OK;
     // the instability test of src/m_diag.F90:169-173 on the moments just returned (all cells): what
     // the flag stands for, counted for the message
@@ -1053,7 +1052,8 @@ int upload_field(lbm_ctx* c, int nv, const void* host, int realkind, DevBuf* to)
         if (int rc = dev_alloc(c, to[q], (size_t)c->lay.cplane * c->ops->real_bytes)) return rc;
         p[q] = to[q].p;
     }
-    HIPCHK(c, hipMemcpyAsync(c->stage.p, host, n, hipMemcpyHostToDevice, c->stream));
+    const HostPart part{const_cast<void*>(host), 0, n};
+    if (int rc = copy_in(c, c->stage.p, &part, 1)) return rc;
     HIPCHK(c, c->ops->field_in(c->lay, nv, c->stage.p, realkind, p, c->stream));
     HIPCHK(c, hipStreamSynchronize(c->stream));
     return LBM_OK;

@@ -1,0 +1,27 @@
+// Arrays of the caller's ordinary (pageable) memory from and to device memory.
+#pragma once
+
+#include <cstddef>
+
+#include "ctx.h"
+
+namespace lbm_host {
+
+// A piece of a device range: bytes at offset, at host in the caller's memory (nullptr: not wanted).
+struct HostPart {
+    void* host;
+    size_t offset, bytes;
+};
+
+// Copies the parts of the device range that starts at dev, in stream order, and returns when they are
+// there.  Parts are in ascending order and do not overlap.
+int copy_out(lbm_ctx* c, const void* dev, const HostPart* parts, int n);
+// The other way; returns when the caller's arrays have been read.  The parts cover the range.
+int copy_in(lbm_ctx* c, void* dev, const HostPart* parts, int n);
+
+// The page-locked buffers that the copies go through are the process's: allocated by the first copy,
+// freed when the last context goes.
+void transfer_retain();
+void transfer_release();
+
+}  // namespace lbm_host
