@@ -470,7 +470,7 @@ __global__ void __launch_bounds__(256) adjoint_step_kernel(const StepArgs<typena
     }
 }
 
-// Reverse of the inflow/outflow pass (inflow_cell) of step n on the adjoint buffer lam of X(n).
+// Reverse of the inflow/outflow pass (fold_inflow, boundary_kernel) of step n on the adjoint buffer lam of X(n).
 // gS: FP64 accumulators of d/d uvel_shear per (j,k) (j fastest).
 template <int Q, class C>
 __global__ void __launch_bounds__(64) adjoint_inflow_kernel(Layout L, typename C::raw* lam, typename C::real utime, typename C::real cosd,

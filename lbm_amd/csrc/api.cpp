@@ -217,31 +217,6 @@ EdgeList edge_list(const lbm_desc& d) {
     return e;
 }
 
-// Ghost cells read by a closed-face pass while holding the first periodic pass's copy of a cell
-// that an earlier closed pass of the same call has rewritten (pass order i, j, k;
-// src/m_boundarycond.F90:69-255).  For the k faces: tangential (i, j) ghosts where one of i, j is
-// periodic and the other closed; for the j faces: (i, k) ghosts with k periodic and i closed.
-void snap_lists(const lbm_desc& d, SnapList& sk, SnapList& sj) {
-    sk = SnapList{};
-    sj = SnapList{};
-    const bool ci = d.ibnd > 10, cj = d.jbnd > 10, ck = d.kbnd > 10;
-    const bool pi = d.ibnd == 0, pj = d.jbnd == 0, pk = d.kbnd == 0;
-    if (ck && ((pi && cj) || (ci && pj)))
-        for (int a : {0, d.nx + 1})
-            for (int b : {0, d.ny + 1})
-                for (int c : {1, d.nz}) {
-                    sk.g[sk.n][0] = a; sk.g[sk.n][1] = b; sk.g[sk.n][2] = c;
-                    ++sk.n;
-                }
-    if (cj && pk && ci)
-        for (int a : {0, d.nx + 1})
-            for (int b : {1, d.ny})
-                for (int c : {0, d.nz + 1}) {
-                    sj.g[sj.n][0] = a; sj.g[sj.n][1] = b; sj.g[sj.n][2] = c;
-                    ++sj.n;
-                }
-}
-
 double utime_at(const lbm_ctx* c, int it) {
     if (!c->ut_series.empty() && it >= c->series_lo && it <= c->series_hi) return c->ut_series[it - c->series_lo];
     return c->uini;
@@ -337,34 +312,32 @@ int step_buffers(lbm_ctx* c, const void* src, void* dst, int it) {
 // skip_dir: a closed axis whose face pass the step kernel has already performed.
 int boundary(lbm_ctx* c, void* f1, const void* f2, int it, int skip_dir, bool skip_inflow, bool timed) {
     const lbm_desc& d = c->d;
-    const Layout& L = c->lay;
-    int a1, a2, b1, b2, k1, k2;
-    opts_of(d.ibnd, &a1, &a2);
-    opts_of(d.jbnd, &b1, &b2);
-    opts_of(d.kbnd, &k1, &k2);
-    // timed: bracket the boundary kernels with events, if this step launches any
-    timed = timed && (c->snap_k.n || c->snap_j.n || (a1 && skip_dir != 0) || (b1 && skip_dir != 1) ||
-                      (k1 && skip_dir != 2) || (d.ibnd == 1 && !skip_inflow));
+    BoundaryHost h{};
+    h.f1 = f1;
+    h.f2 = f2;
+    const int codes[3] = {d.ibnd, d.jbnd, d.kbnd};
+    bool any = false;
+    for (int a = 0; a < 3; ++a) {
+        if (a == skip_dir) continue;
+        opts_of(codes[a], &h.opt_lo[a], &h.opt_hi[a]);
+        any = any || h.opt_lo[a] != 0;
+    }
+    h.inflow = d.ibnd == 1;
+    h.do_inflow = h.inflow && !skip_inflow;
+    if (!any && !h.do_inflow) return LBM_OK;
+    h.edges = edge_list(d);
+    if (h.do_inflow) {
+        h.shear = c->shear.p;
+        h.rho0 = d.rho0;
+        inflow_values(c, it, &h.utime, &h.cosd, &h.sind);
+    }
+    // timed: bracket the launch with events
     hipEvent_t e0 = nullptr;
     if (timed) {
         e0 = next_event(c, c->ev_bc, c->n_bc_ev);
         if (e0) hipEventRecord(e0, c->stream);
     }
-    const SnapList none{};
-    char* snap = static_cast<char*>(c->snap.p);
-    const size_t half = (size_t)8 * d.q * c->ops->raw_bytes;
-    if (c->snap_k.n) HIPCHK(c, c->ops->snapshot(L, f1, snap, c->snap_k, c->stream));
-    if (c->snap_j.n) HIPCHK(c, c->ops->snapshot(L, f1, snap + half, c->snap_j, c->stream));
-    if (a1 && skip_dir != 0) HIPCHK(c, c->ops->closed(L, f1, f2, 0, a1, a2, nullptr, none, c->stream));
-    if (b1 && skip_dir != 1) HIPCHK(c, c->ops->closed(L, f1, f2, 1, b1, b2, snap + half, c->snap_j, c->stream));
-    if (k1 && skip_dir != 2) HIPCHK(c, c->ops->closed(L, f1, f2, 2, k1, k2, snap, c->snap_k, c->stream));
-    const EdgeList e = edge_list(d);
-    if (e.n) HIPCHK(c, c->ops->edges(L, f1, f2, e, c->stream));
-    if (d.ibnd == 1 && !skip_inflow) {
-        double ut, cs, sn;
-        inflow_values(c, it, &ut, &cs, &sn);
-        HIPCHK(c, c->ops->inflow(L, f1, c->shear.p, ut, cs, sn, d.rho0, c->stream));
-    }
+    HIPCHK(c, c->ops->boundary(c->lay, h, c->stream));
     if (timed && e0) {
         hipEvent_t e1 = next_event(c, c->ev_bc, c->n_bc_ev);
         if (e1) hipEventRecord(e1, c->stream);
@@ -539,12 +512,6 @@ int lbm_create(const lbm_desc* desc, lbm_ctx** out) {
         if ((e = hipMalloc(&c->buf[b], c->buf_bytes)) != hipSuccess) return bail(e, "hipMalloc(populations)");
     for (int b = 0; b < 2; ++b)
         if ((e = hipMemsetAsync(c->buf[b], 0, c->buf_bytes, c->stream)) != hipSuccess) return bail(e, "hipMemset");
-    snap_lists(d, c->snap_k, c->snap_j);
-    if (c->snap_k.n || c->snap_j.n) {
-        const size_t sb = (size_t)16 * d.q * ops->raw_bytes;
-        if ((e = hipMalloc(&c->snap.p, sb)) != hipSuccess) return bail(e, "hipMalloc(snapshot)");
-        c->snap.n = sb;
-    }
     if (d.store_tau && d.ivreman) {
         const size_t tb = (size_t)c->lay.cplane * ops->real_bytes;
         if ((e = hipMalloc(&c->tau.p, tb)) != hipSuccess) return bail(e, "hipMalloc(tau)");
@@ -572,7 +539,7 @@ int lbm_destroy(lbm_ctx* c) {
         if (c->buf[b]) hipFree(c->buf[b]);
     DevBuf* all[] = {&c->ablvisc, &c->shear, &c->solid, &c->turb[0], &c->turb[1], &c->turb[2], &c->force[0],
                      &c->force[1], &c->force[2], &c->tau, &c->ext[0], &c->ext[1], &c->ext[2], &c->ext[3],
-                     &c->stage, &c->partial, &c->snap, &c->t_rot, &c->t_theta, &c->t_blade, &c->t_nfoil,
+                     &c->stage, &c->partial, &c->t_rot, &c->t_theta, &c->t_blade, &c->t_nfoil,
                      &c->t_nang, &c->t_foil, &c->t_pts, &c->t_box, &c->theta, &c->adj_ck, &c->adj_snaps,
                      &c->adj_lam, &c->adj_gF, &c->adj_gS, &c->adj_acc};
     for (DevBuf* b : all) dev_free(*b);

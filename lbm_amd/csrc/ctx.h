@@ -42,8 +42,7 @@ struct lbm_ctx {
     bool ghost_raw[2] = {true, true};
     bool use_ext = false;          // first collision uses the moments given at initialisation
     // inputs
-    lbm_host::DevBuf ablvisc, shear, solid, turb[3], force[3], tau, ext[4], stage, partial, snap;
-    lbm::SnapList snap_k{}, snap_j{};
+    lbm_host::DevBuf ablvisc, shear, solid, turb[3], force[3], tau, ext[4], stage, partial;
     int solid_wpr = 0;
     bool has_solid = false, has_turb = false, has_force = false;
     int nrturb = 0;

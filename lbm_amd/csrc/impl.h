@@ -8,8 +8,8 @@
 
 namespace lbm {
 
-struct EdgeSpec;
-
+// Ghost edges (kind 0, along axis t, len cells) and corners (kind 1) of closed axes: the ghost g, the
+// outward direction of each closed axis, the factors of the mirrored velocity.
 struct EdgeList {
     int n;
     int len[20];
@@ -20,13 +20,15 @@ struct EdgeList {
     int mir[20][3];
 };
 
-// Ghost cells that a closed-face pass reads while they hold a copy made by the reference's first
-// periodic pass (src/m_boundarycond.F90:69-159) of a cell that an earlier closed pass of the same
-// call has since rewritten.  g holds the ghost coordinates as read; the snapshot of the copied
-// cell is taken before the closed passes.
-struct SnapList {
-    int n;
-    int g[8][3];
+// The boundary passes of one step that the step kernel does not perform.
+struct BoundaryHost {
+    void* f1;
+    const void* f2;
+    int opt_lo[3], opt_hi[3];   // wall options of the closed axes (0: not closed, or not this launch's)
+    int inflow, do_inflow;      // i has inflow/outflow planes; they are this launch's
+    const void* shear;          // uvel_shear(nz) (compute type)
+    double utime, cosd, sind, rho0;
+    EdgeList edges;
 };
 
 // Everything the host passes to one step-kernel launch, in double; converted to the compute
@@ -128,12 +130,7 @@ inline int objective_blocks(const AdjBox& b) {
 
 struct Ops {
     hipError_t (*step)(const Layout&, const StepHost&, hipStream_t);
-    hipError_t (*closed)(const Layout&, void* f1, const void* f2, int dir, int opt_lo, int opt_hi, const void* snap,
-                         const SnapList&, hipStream_t);
-    hipError_t (*snapshot)(const Layout&, const void* f1, void* snap, const SnapList&, hipStream_t);
-    hipError_t (*edges)(const Layout&, void* f1, const void* f2, const EdgeList&, hipStream_t);
-    hipError_t (*inflow)(const Layout&, void* f1, const void* shear, double utime, double cosd, double sind,
-                         double rho0, hipStream_t);
+    hipError_t (*boundary)(const Layout&, const BoundaryHost&, hipStream_t);
     hipError_t (*aos_in)(const Layout&, const void* aos, int realkind, void* dstA, void* dstB, hipStream_t);
     hipError_t (*state_out)(const Layout&, const void* cur, const void* gsrc, int stream_interior, int ghost_raw,
                             void* aos, int realkind, hipStream_t);

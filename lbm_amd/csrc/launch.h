@@ -158,13 +158,6 @@ struct Launch {
         }
     }
 
-    static hipError_t snapshot(const Layout& L, const void* f1, void* snap, const SnapList& sl, hipStream_t s) {
-        if (sl.n == 0) return hipSuccess;
-        hipLaunchKernelGGL((bc_snapshot_kernel<Q, C>), dim3(1), dim3(256), 0, s, L, f1, snap, sl);
-        return hipGetLastError();
-    }
-
-    // side 0 or 1, or 2: both (side 0's halo first in buf)
     static hipError_t ghost_copy(const Layout& L, const void* src, void* dst, hipStream_t s) {
         const int per[3] = {L.per_i, L.per_j, L.per_k};
         const int n1 = L.n(L.ax1), n2 = L.n(L.ax2);
@@ -233,40 +226,38 @@ struct Launch {
         return hipGetLastError();
     }
 
-    static hipError_t closed(const Layout& L, void* f1, const void* f2, int dir, int opt_lo, int opt_hi,
-                             const void* snap, const SnapList& sl, hipStream_t s) {
-        // tangential axes in storage order: threads run along the first
-        const int order[3] = {L.ax0, L.ax1, L.ax2};
-        int t[2], q = 0;
-        for (int a = 0; a < 3; ++a)
-            if (order[a] != dir) t[q++] = order[a];
-        const dim3 block(64, 4, 1);
-        const dim3 grid((L.n(t[0]) + 63) / 64, (L.n(t[1]) + 3) / 4, 1);
-        if (dir == 0) hipLaunchKernelGGL((bc_closed_kernel<Q, C, 0>), grid, block, 0, s, L, f1, f2, opt_lo, opt_hi, t[0], t[1], snap, sl);
-        else if (dir == 1) hipLaunchKernelGGL((bc_closed_kernel<Q, C, 1>), grid, block, 0, s, L, f1, f2, opt_lo, opt_hi, t[0], t[1], snap, sl);
-        else hipLaunchKernelGGL((bc_closed_kernel<Q, C, 2>), grid, block, 0, s, L, f1, f2, opt_lo, opt_hi, t[0], t[1], snap, sl);
-        return hipGetLastError();
-    }
-
-    static hipError_t edges(const Layout& L, void* f1, const void* f2, const EdgeList& e, hipStream_t s) {
-        if (e.n == 0) return hipSuccess;
-        int mx = 1;
-        for (int q = 0; q < e.n; ++q) mx = e.len[q] > mx ? e.len[q] : mx;
-        const dim3 block(64, 1, 1);
-        const dim3 grid((mx + 63) / 64, e.n, 1);
-        hipLaunchKernelGGL((bc_edges_kernel<Q, C>), grid, block, 0, s, L, f1, f2, e);
-        return hipGetLastError();
-    }
-
-    static hipError_t inflow(const Layout& L, void* f1, const void* shear, double utime, double cosd, double sind,
-                             double rho0, hipStream_t s) {
-        // threads along j or k, whichever is stored first
-        const int jfast = (L.ax0 == 1) || (L.ax0 == 0 && L.ax1 == 1);
-        const int nx_ = jfast ? L.ny : L.nz, ny_ = jfast ? L.nz : L.ny;
-        const dim3 block(64, 4, 1);
-        const dim3 grid((nx_ + 63) / 64, (ny_ + 3) / 4, 1);
-        hipLaunchKernelGGL((bc_inflow_kernel<Q, C>), grid, block, 0, s, L, f1, static_cast<const R*>(shear), (R)utime,
-                           (R)cosd, (R)sind, (R)rho0, jfast);
+    static hipError_t boundary(const Layout& L, const BoundaryHost& h, hipStream_t s) {
+        BoundaryArgs<R> a{};
+        a.lay = L;
+        a.f1 = h.f1;
+        a.f2 = h.f2;
+        a.inflow = h.inflow;
+        long long blocks = 0;
+        for (int d = 0; d < 3; ++d) {
+            a.ta[d] = L.ax0 != d ? L.ax0 : L.ax1;
+            const int t1 = 3 - d - a.ta[d];
+            const long long area = ((long long)L.n(a.ta[d]) * L.n(t1) + 255) / 256;
+            a.face[d] = h.opt_lo[d] != 0;
+            a.opt_lo[d] = h.opt_lo[d];
+            a.opt_hi[d] = h.opt_hi[d];
+            a.face_blocks[d] = a.face[d] ? (int)(area * 2 * Outgoing<Q>::count) : 0;
+            blocks += a.face_blocks[d];
+            if (d == 0 && h.do_inflow) {
+                a.inflow_blocks = (int)(area * Q);
+                blocks += a.inflow_blocks;
+            }
+        }
+        a.shear = static_cast<const R*>(h.shear);
+        a.utime = (R)h.utime;
+        a.cosd = (R)h.cosd;
+        a.sind = (R)h.sind;
+        a.rho0 = (R)h.rho0;
+        a.edges = h.edges;
+        long long along = 0;
+        for (int q = 0; q < h.edges.n; ++q) along += 3LL * h.edges.len[q];
+        blocks += (along + 255) / 256;
+        if (blocks == 0) return hipSuccess;
+        hipLaunchKernelGGL((boundary_kernel<Q, C>), dim3((unsigned)blocks), dim3(256), 0, s, a);
         return hipGetLastError();
     }
 
@@ -447,7 +438,7 @@ struct Launch {
     }
 
     static const Ops* ops() {
-        static const Ops o = {&step, &closed, &snapshot, &edges, &inflow, &aos_in, &state_out, &moments_out,
+        static const Ops o = {&step, &boundary, &aos_in, &state_out, &moments_out,
                               &averages_out, &field_in, &feq_init, &totals, &average,
                               sizeof(MemberTab<R>), &ens_pack, &ens_step,
                               kAdj ? &adj_step : nullptr, kAdj ? &adj_inflow : nullptr, kAdj ? &adj_face : nullptr,
