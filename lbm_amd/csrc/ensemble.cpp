@@ -36,9 +36,9 @@ struct lbm_ens {
     int block = 256;
     int bpc = 0;                   // persistent grid of bpc blocks per CU; 0: one block per tile
     // device tables and their host images
-    DevBuf tab, start, vals, clock, backup;
+    DevBuf tab, owner, vals, clock, backup;
     std::vector<unsigned char> h_tab, h_vals;
-    std::vector<int> h_start;
+    std::vector<int> h_owner;
     int h_clock[3] = {0, 0, 0};
     EnsLaunch L{};
     // captured graphs by number of steps, valid for the launch in `key`
@@ -102,7 +102,7 @@ int build_tables(lbm_ens* e) {
     const int n = (int)e->mem.size();
     const size_t mb = e->ops->member_bytes;
     e->h_tab.assign(mb * n, 0);
-    e->h_start.assign(n, 0);
+    std::vector<int> own;
     long long total = 0;
     for (int m = 0; m < n; ++m) {
         lbm_ctx* c = e->mem[m];
@@ -118,22 +118,25 @@ int build_tables(lbm_ens* e) {
         mh.shear = c->shear.p;
         mh.rho0 = c->d.rho0;
         mh.inflow = c->d.ibnd == 1;
-        int tiles = 0;
-        e->ops->ens_pack(mh, e->block, e->h_tab.data() + mb * m, &tiles);
-        e->h_start[m] = (int)total;
+        long long tiles = 0;
+        e->ops->ens_pack(mh, e->block, (int)total, e->h_tab.data() + mb * m, &tiles);
         total += tiles;
+        if (total >= (1LL << 31)) return efail(e, LBM_EINVAL, "ensemble too large for 32-bit tile indices");
+        own.resize((size_t)total, m);
     }
-    if (total >= (1LL << 31)) return efail(e, LBM_EINVAL, "ensemble too large for 32-bit tile indices");
     bool moved = false;
     if (int rc = ealloc(e, e->tab, mb * n, &moved)) return rc;
-    if (int rc = ealloc(e, e->start, sizeof(int) * n, &moved)) return rc;
+    if (int rc = ealloc(e, e->owner, sizeof(int) * own.size(), &moved)) return rc;
     if (int rc = ealloc(e, e->clock, sizeof(e->h_clock), &moved)) return rc;
     if (int rc = ealloc(e, e->vals, (size_t)kChunk * n * 3 * e->ops->real_bytes, &moved)) return rc;
     EHIP(e, hipMemcpyAsync(e->tab.p, e->h_tab.data(), mb * n, hipMemcpyHostToDevice, e->stream));
-    EHIP(e, hipMemcpyAsync(e->start.p, e->h_start.data(), sizeof(int) * n, hipMemcpyHostToDevice, e->stream));
+    if (moved || own != e->h_owner) {
+        e->h_owner.swap(own);
+        EHIP(e, hipMemcpyAsync(e->owner.p, e->h_owner.data(), sizeof(int) * e->h_owner.size(), hipMemcpyHostToDevice, e->stream));
+    }
     EnsLaunch& L = e->L;
     L.tab = e->tab.p;
-    L.start = static_cast<const int*>(e->start.p);
+    L.owner = static_cast<const int*>(e->owner.p);
     L.nmem = n;
     L.total = (int)total;
     L.block = e->block;
@@ -143,7 +146,7 @@ int build_tables(lbm_ens* e) {
     L.bgk3 = e->bgk3;
     L.hrr = e->hrr;
     L.vre = e->vre;
-    std::vector<long long> key = {(long long)(size_t)L.tab, (long long)(size_t)L.start, L.nmem, L.total, L.block,
+    std::vector<long long> key = {(long long)(size_t)L.tab, (long long)(size_t)L.owner, L.nmem, L.total, L.block,
                                   L.grid, (long long)(size_t)L.vals, (long long)(size_t)L.clock};
     if (moved || key != e->key) {
         drop_graphs(e);
@@ -160,7 +163,8 @@ int graph_for(lbm_ens* e, int steps, hipGraphExec_t* out) {
     }
     EHIP(e, hipStreamBeginCapture(e->stream, hipStreamCaptureModeThreadLocal));
     hipError_t le = hipSuccess;
-    for (int s = 0; s < steps && le == hipSuccess; ++s) le = e->ops->ens_step(e->L, e->stream);
+    for (int s = 0; s < steps && le == hipSuccess; ++s) le = e->ops->ens_step(e->L, s, e->stream);
+    if (le == hipSuccess) le = e->ops->ens_tick(e->L, steps, e->stream);
     hipGraph_t g = nullptr;
     const hipError_t ce = hipStreamEndCapture(e->stream, &g);
     if (le != hipSuccess) {
@@ -304,7 +308,7 @@ int lbm_ensemble_destroy(lbm_ens* e) {
     e->tag = 0;
     if (e->stream) hipStreamSynchronize(e->stream);
     drop_graphs(e);
-    for (DevBuf* b : {&e->tab, &e->start, &e->vals, &e->clock, &e->backup}) dev_free(*b);
+    for (DevBuf* b : {&e->tab, &e->owner, &e->vals, &e->clock, &e->backup}) dev_free(*b);
     for (hipEvent_t x : e->ev) hipEventDestroy(x);
     for (hipEvent_t x : e->ev_mem)
         if (x) hipEventDestroy(x);

@@ -79,14 +79,13 @@ struct MemberHost {
     int inflow;            // inflow/outflow planes of i (folded into the batched step)
 };
 
-// One batched step: the step kernel over every member's tiles (faces and inflow planes folded),
-// the clock tick.
+// One batched step: the step kernel over every member's tiles (faces and inflow planes folded).
 struct EnsLaunch {
     const void* tab;                 // device MemberTab<R>[nmem]
-    const int* start;                // device tile starts [nmem]
+    const int* owner;                // device member of each tile [total]
     int nmem, total, block, grid;
     const void* vals;                // device (utime, cos, sin)[steps of the table][nmem]
-    int* clock;                      // device {it, steps since set, table's first step}
+    int* clock;                      // device {it of a graph's first step, steps since set, table's first step}
     int bgk3, hrr, vre;
 };
 
@@ -149,8 +148,9 @@ struct Ops {
     hipError_t (*average)(const Layout&, const void* cur, int stream_interior, void* avg, hipStream_t);
     // ensembles
     size_t member_bytes;   // sizeof(MemberTab<R>)
-    void (*ens_pack)(const MemberHost&, int block, void* out, int* tiles);
-    hipError_t (*ens_step)(const EnsLaunch&, hipStream_t);
+    void (*ens_pack)(const MemberHost&, int block, int start, void* out, long long* tiles);
+    hipError_t (*ens_step)(const EnsLaunch&, int sub, hipStream_t);   // step clock + sub
+    hipError_t (*ens_tick)(const EnsLaunch&, int steps, hipStream_t);
     // adjoint (nullptr for the 16-bit storage codecs)
     hipError_t (*adj_step)(const Layout&, const StepHost&, const void* lam_y, void* lam_x, const AdjBox&, double kappa,
                            int coll, double* gF, hipStream_t);

@@ -322,7 +322,7 @@ struct Launch {
     }
 
     // ---- ensembles
-    static void ens_pack(const MemberHost& m, int block, void* out, int* tiles) {
+    static void ens_pack(const MemberHost& m, int block, int start, void* out, long long* tiles) {
         const Layout& L = m.lay;
         MemberTab<R> t{};
         t.a = args_of(L, m.h);
@@ -334,37 +334,43 @@ struct Launch {
         t.nrturb = m.turb[0] ? m.nrturb : 0;
         t.slice = L.ny * L.nz;
         for (int q = 0; q < 3; ++q) t.turb[q] = static_cast<const R*>(m.turb[q]);
-        t.n0 = L.n(L.ax0);
-        const long long plane = (long long)L.n(L.ax0) * L.n(L.ax1);
+        constexpr int W = kSegment<typename C::raw>;
+        t.seg_row = (L.n(L.ax0) + W - 1) / W;
+        const long long plane = (long long)t.seg_row * W * L.n(L.ax1);
         t.tiles_plane = (int)((plane + block - 1) / block);
+        t.start = start;
         t.a.inflow_fold = m.inflow;
         t.a.shear = static_cast<const R*>(m.shear);
         t.a.rho0 = (R)m.rho0;
         std::memcpy(out, &t, sizeof(t));
-        *tiles = t.tiles_plane * L.n(L.ax2);
+        *tiles = (long long)t.tiles_plane * L.n(L.ax2);
     }
 
     template <bool B3, bool H, bool V>
-    static void ens_step_t(const EnsLaunch& e, hipStream_t s) {
+    static void ens_step_t(const EnsLaunch& e, int sub, hipStream_t s) {
         if constexpr (kNT)
             hipLaunchKernelGGL((step_kernel_batch<Q, C, B3, H, V>), dim3(e.grid), dim3(e.block), 0, s,
-                               static_cast<const MemberTab<R>*>(e.tab), e.start, e.nmem, e.total,
-                               static_cast<const R*>(e.vals), e.clock);
+                               static_cast<const MemberTab<R>*>(e.tab), e.owner, e.nmem, e.total,
+                               static_cast<const R*>(e.vals), e.clock, sub);
     }
 
-    static hipError_t ens_step(const EnsLaunch& e, hipStream_t s) {
+    static hipError_t ens_step(const EnsLaunch& e, int sub, hipStream_t s) {
         const int key = (e.bgk3 ? 4 : 0) | (e.hrr ? 2 : 0) | (e.vre ? 1 : 0);
         switch (key) {
-            case 0: ens_step_t<false, false, false>(e, s); break;
-            case 1: ens_step_t<false, false, true>(e, s); break;
-            case 2: ens_step_t<false, true, false>(e, s); break;
-            case 3: ens_step_t<false, true, true>(e, s); break;
-            case 4: ens_step_t<true, false, false>(e, s); break;
-            case 5: ens_step_t<true, false, true>(e, s); break;
-            case 6: ens_step_t<true, true, false>(e, s); break;
-            default: ens_step_t<true, true, true>(e, s); break;
+            case 0: ens_step_t<false, false, false>(e, sub, s); break;
+            case 1: ens_step_t<false, false, true>(e, sub, s); break;
+            case 2: ens_step_t<false, true, false>(e, sub, s); break;
+            case 3: ens_step_t<false, true, true>(e, sub, s); break;
+            case 4: ens_step_t<true, false, false>(e, sub, s); break;
+            case 5: ens_step_t<true, false, true>(e, sub, s); break;
+            case 6: ens_step_t<true, true, false>(e, sub, s); break;
+            default: ens_step_t<true, true, true>(e, sub, s); break;
         }
-        hipLaunchKernelGGL((clock_tick_kernel<Q, C>), dim3(1), dim3(64), 0, s, e.clock);
+        return hipGetLastError();
+    }
+
+    static hipError_t ens_tick(const EnsLaunch& e, int steps, hipStream_t s) {
+        hipLaunchKernelGGL((clock_tick_kernel<Q, C>), dim3(1), dim3(64), 0, s, e.clock, steps);
         return hipGetLastError();
     }
 
@@ -440,7 +446,7 @@ struct Launch {
     static const Ops* ops() {
         static const Ops o = {&step, &boundary, &aos_in, &state_out, &moments_out,
                               &averages_out, &field_in, &feq_init, &totals, &average,
-                              sizeof(MemberTab<R>), &ens_pack, &ens_step,
+                              sizeof(MemberTab<R>), &ens_pack, &ens_step, &ens_tick,
                               kAdj ? &adj_step : nullptr, kAdj ? &adj_inflow : nullptr, kAdj ? &adj_face : nullptr,
                               &objective, &halo_pack, &halo_unpack, &ghost_copy, &turb_step, (int)sizeof(R),
                               (int)sizeof(typename C::raw)};
