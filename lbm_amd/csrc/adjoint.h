@@ -470,7 +470,7 @@ __global__ void __launch_bounds__(256) adjoint_step_kernel(const StepArgs<typena
     }
 }
 
-// Reverse of the inflow/outflow pass (fold_inflow, boundary_kernel) of step n on the adjoint buffer lam of X(n).
+// Reverse of the inflow/outflow pass (fold_boundaries, boundary_kernel) of step n on the adjoint buffer lam of X(n).
 // gS: FP64 accumulators of d/d uvel_shear per (j,k) (j fastest).
 template <int Q, class C>
 __global__ void __launch_bounds__(64) adjoint_inflow_kernel(Layout L, typename C::raw* lam, typename C::real utime, typename C::real cosd,
@@ -505,7 +505,7 @@ __global__ void __launch_bounds__(64) adjoint_inflow_kernel(Layout L, typename C
     if (gS != nullptr) gS[(size_t)(k - 1) * L.ny + (j - 1)] += (double)(s * utime);
 }
 
-// Reverse of the closed-face pass of axis D (fold_closed_face) of step n: lam_y adjoint of X(n),
+// Reverse of the closed-face pass of axis D (fold_boundaries) of step n: lam_y adjoint of X(n),
 // lam_x adjoint of X(n-1).  One thread per ghost cell of the two faces (tangential coordinates
 // interior), t0/t1 the tangential axes.
 template <int Q, class C>

@@ -424,73 +424,41 @@ __host__ __device__ __forceinline__ void collide_cell(const StepArgs<typename C:
     collide_cell<Q, C, BGK3, HRR, VRE, false>(a, rv, CellAux<typename C::real>{}, i, j, k, ca, cb, cc, oc, true, dev, tau_out);
 }
 
-// The closed-face pass of axis D (src/m_boundary_{i,j,k}_closed_kernel.F90) performed by the
-// step kernel for the cells next to the walls, when D is the only closed axis (the other axes
-// periodic, or i carrying the inflow/outflow planes, whose kernel runs after this one).  For
-// ghost cell G of the face and outgoing l the reference sets
-//   f1(m, G) = f2(l, G)                 (m = l reflected: normal negated, tangential * opt)
-//   f1(l, G) = f1(l, G - c_l tangentially, on the wall plane).
-// The cell x above G does the first; the second is pushed by the cell G - c_l that computed
-// the value (periodic tangential axes wrapped), or, when G - c_l is a stored ghost of the
-// inflow axis, copied by x from that ghost (still holding its value from before this step).
-template <int Q, class C>
-__device__ __forceinline__ void fold_closed_face(const StepArgs<typename C::real>& a, int i, int j, int k,
-                                                 const typename C::real (&dev)[Q]) {
-    using Lt = Lattice<Q>;
-    using raw = typename C::raw;
-    const Layout& L = a.lay;
-    const int D = a.fold_dir;
-    const int x[3] = {i, j, k};
-    const int n[3] = {L.nx, L.ny, L.nz};
-    const int per[3] = {L.per_i, L.per_j, L.per_k};
-    const raw* __restrict__ f2 = static_cast<const raw*>(a.src);
-    raw* __restrict__ f1 = static_cast<raw*>(a.dst);
-#pragma unroll
-    for (int side = 0; side < 2; ++side) {
-        const int plane = side ? n[D] : 1;
-        if (x[D] != plane) continue;
-        const int ghost = side ? n[D] + 1 : 0;
-        const int opt = side ? a.fold_opt_hi : a.fold_opt_lo;
-        int g[3] = {i, j, k};
-        g[D] = ghost;
-        const int og = L.cell(g[0], g[1], g[2]);
-#pragma unroll
-        for (int l = 0; l < Q; ++l) {
-            const int cn = Lt::c(l, D);
-            if (!(side ? cn > 0 : cn < 0)) continue;
-            const int m = opt < 0 ? mirror<Q>(l, D, -1) : mirror<Q>(l, D, +1);
-            f1[(size_t)m * L.plane + og] = f2[(size_t)l * L.plane + og];
-            // push: the ghost this population streams to
-            int t[3], s[3];
-            bool push = true, from_inflow = false, from_halo = false;
-#pragma unroll
-            for (int d = 0; d < 3; ++d) {
-                if (d == D) { t[d] = ghost; s[d] = plane; continue; }
-                const int cd = Lt::c(l, d);
-                t[d] = x[d] + cd;
-                s[d] = x[d] - cd;
-                if (per[d]) {
-                    t[d] = Layout::wrap(t[d], n[d], 1);
-                    s[d] = Layout::wrap(s[d], n[d], 1);
-                } else {
-                    if (t[d] < 1 || t[d] > n[d]) push = false;
-                    if (s[d] < 1 || s[d] > n[d]) {
-                        if (d == a.halo_dir) from_halo = true;
-                        else from_inflow = true;
-                    }
-                }
-            }
-            if (push) f1[(size_t)l * L.plane + L.cell(t[0], t[1], t[2])] = C::template enc_dep<Q>(dev[l], l);
-            // G - c_l outside the face's range.  On a halo plane only: the neighbour's value of this
-            // step, pushed by that halo's unpack.  On the inflow axis only: the ghost's value from
-            // before this step, copied by the cell that rewrites the ghost when the inflow planes are
-            // folded too, else here.  On both (the inflow ghost of a halo plane): the value that
-            // ghost holds now, the neighbour's inflow ghost from before this step.
-            if (from_inflow && (from_halo || !a.inflow_fold))
-                f1[(size_t)l * L.plane + og] = f1[(size_t)l * L.plane + L.cell(s[0], s[1], s[2])];
-        }
+// Directions by run-time values, from packed constants (scalar shifts and masks).
+template <int Q>
+struct Outgoing {
+    // populations with c_d > 0 (side 1) or < 0 (side 0), in lattice order, five bits each
+    static constexpr int count = Q == 27 ? 9 : 5;
+    static constexpr unsigned long long pack(int d, int side) {
+        unsigned long long p = 0;
+        int n = 0;
+        for (int l = 0; l < Q; ++l)
+            if (Lattice<Q>::c(l, d) == (side ? 1 : -1)) p |= (unsigned long long)l << (5 * n++);
+        return p;
     }
-}
+    __device__ static __forceinline__ int pop(int d, int side, int q) {
+        constexpr unsigned long long k[6] = {pack(0, 0), pack(0, 1), pack(1, 0), pack(1, 1), pack(2, 0), pack(2, 1)};
+        const unsigned long long p = d == 0 ? (side ? k[1] : k[0]) : d == 1 ? (side ? k[3] : k[2]) : (side ? k[5] : k[4]);
+        return (int)((p >> (5 * q)) & 31ull);
+    }
+};
+template <int Q>
+struct Direction {
+    // the direction with velocity (x, y, z), 31 if the lattice has none
+    static constexpr unsigned long long pack(int part) {
+        unsigned long long p = 0;
+        for (int e = 0; e < 9; ++e) {
+            const int l = Lattice<Q>::find(part - 1, e / 3 - 1, e % 3 - 1);
+            p |= (unsigned long long)(l < 0 ? 31 : l) << (5 * e);
+        }
+        return p;
+    }
+    __device__ static __forceinline__ int find(int x, int y, int z) {
+        constexpr unsigned long long k[3] = {pack(0), pack(1), pack(2)};
+        const unsigned long long p = x < 0 ? k[0] : x == 0 ? k[1] : k[2];
+        return (int)((p >> (5 * (3 * (y + 1) + z + 1))) & 31ull);
+    }
+};
 
 // Inflow ghost value (src/m_boundary_i_inflow_kernel.F90:61-74) from population l of cell (1, j, k):
 // f_l - 2 w_l rho0 (c_x u cos(udir) + c_y u sin(udir)) / cs^2.
@@ -506,47 +474,140 @@ __host__ __device__ __forceinline__ R inflow_ghost_value(R f, int l, R uu, R cos
     return f - R(2) * wl * rho0 * (cxl * uu * cosd + cyl * uu * sind) / cs2;
 }
 
-// The inflow/outflow pass for the ghost row (j, k) of i, performed by the cell (i, j, k) with
-// i = 1 (inflow ghost i = 0) or i = nx (outflow ghost i = nx+1, a copy of the cell) from the
-// values it has just stored.  When the closed face of fold_dir is folded as well, the face pass
-// reads this ghost's value from before the step (f1(l, G - c_l) on the wall plane, G - c_l on
-// the inflow axis): those copies are made here, before the ghost is rewritten.
+// The boundary passes performed by the step kernel for its cell (i, j, k) (offset oc in f1, post-collision
+// departures dev), when at most one axis D is closed (the other axes periodic, halo, or i carrying the
+// inflow/outflow planes).
+//
+// Closed face (src/m_boundary_{i,j,k}_closed_kernel.F90): for ghost cell G of the face and outgoing l
+// the reference sets
+//   f1(m, G) = f2(l, G)                 (m = l reflected: normal negated, tangential * opt)
+//   f1(l, G) = f1(l, G - c_l tangentially, on the wall plane).
+// The cell x above G does the first; the second is pushed by the cell G - c_l that computed
+// the value (periodic tangential axes wrapped), or, when G - c_l is a stored ghost of the
+// inflow axis, copied from that ghost (still holding its value from before this step).
+//
+// Inflow/outflow (src/m_boundary_i_inflow_kernel.F90): the ghost row (j, k) of i is written by the cell
+// with i = 1 (inflow ghost i = 0) or i = nx (outflow ghost i = nx+1, a copy of the cell) from the
+// values it has just stored.  The face pass reads this ghost's value from before the step
+// (f1(l, G - c_l) on the wall plane): those copies are made before the ghost is rewritten.
+//
+// All of a cell's loads are issued before the first of its ghost stores: one memory round trip where a
+// copy at a time took up to twelve, each of them behind the stores before it, which was the whole time
+// of a small grid.  (Issued before the cell's own 27 stores instead, they cost 20 registers.)
+// Measured on MI355X, D3Q27 inflow and one closed axis, per step: FP32 60x14x5 11.6 -> 6.6 us,
+// 384x200x128 416 -> 408 us, 384x192x128 351.5 -> 349.7 us; FP16 400x200x100 181 -> 178 us.
+template <int Q, class C, int D, int SIDE>
+__device__ __forceinline__ void fold_face(const StepArgs<typename C::real>& a, int i, int j, int k, int oc, bool at_end,
+                                          const typename C::real (&dev)[Q]) {
+    using raw = typename C::raw;
+    using Lt = Lattice<Q>;
+    constexpr int NO = Outgoing<Q>::count;
+    constexpr unsigned long long out = Outgoing<Q>::pack(D, SIDE);
+    constexpr int T0 = D == 0 ? 1 : 0, T1 = D == 2 ? 1 : 2;   // the axes along the face
+    const Layout& L = a.lay;
+    const int x[3] = {i, j, k};
+    const int n[3] = {L.nx, L.ny, L.nz};
+    const int per[3] = {L.per_i, L.per_j, L.per_k};
+    const int st[3] = {L.si, L.sj, L.sk};
+    const raw* __restrict__ f2 = static_cast<const raw*>(a.src);
+    raw* __restrict__ f1 = static_cast<raw*>(a.dst);
+    const int og = oc + (SIDE ? st[D] : -st[D]);
+    raw above[NO], old[3];
+#pragma unroll
+    for (int q = 0; q < NO; ++q) above[q] = f2[(size_t)((out >> (5 * q)) & 31) * L.plane + og];
+    // the inflow ghost's populations that leave the fluid through the face, by their movement along
+    // the third axis
+    const int ci = i == 1 ? 1 : -1;
+    const bool copy_end = D > 0 && at_end;
+    if (copy_end) {
+#pragma unroll
+        for (int o = 0; o < 3; ++o) {
+            const int l = D == 1 ? Direction<Q>::find(ci, SIDE ? 1 : -1, o - 1) : Direction<Q>::find(ci, o - 1, SIDE ? 1 : -1);
+            if (l < Q) old[o] = f1[(size_t)l * L.plane + oc - ci * st[0]];
+        }
+    }
+    // a step c along each axis of the face: offset, and whether it stays in the face's range
+    int off[2][3];
+    bool ok[2][3];
+#pragma unroll
+    for (int t = 0; t < 2; ++t) {
+        const int d = t ? T1 : T0;
+        const int wrapd = per[d] ? n[d] * st[d] : 0;
+        off[t][0] = -st[d] + (x[d] == 1 ? wrapd : 0);
+        off[t][1] = 0;
+        off[t][2] = st[d] - (x[d] == n[d] ? wrapd : 0);
+        ok[t][0] = per[d] || x[d] > 1;
+        ok[t][1] = true;
+        ok[t][2] = per[d] || x[d] < n[d];
+    }
+#pragma unroll
+    for (int l = 1; l < Q; ++l) {
+        if (Lt::c(l, D) != (SIDE ? 1 : -1)) continue;
+        const int c0 = Lt::c(l, T0) + 1, c1 = Lt::c(l, T1) + 1;
+        if (ok[0][c0] && ok[1][c1])
+            f1[(size_t)l * L.plane + (og + off[0][c0] + off[1][c1])] = C::template enc_dep<Q>(dev[l], l);
+    }
+    const int opt = SIDE ? a.fold_opt_hi : a.fold_opt_lo;
+#pragma unroll
+    for (int q = 0; q < NO; ++q) {
+        const int l = (int)((out >> (5 * q)) & 31);
+        f1[(size_t)(opt < 0 ? mirror<Q>(l, D, -1) : mirror<Q>(l, D, +1)) * L.plane + og] = above[q];
+    }
+    if (copy_end) {
+        constexpr int t = T0 == 0 ? 1 : 0;   // the third axis
+#pragma unroll
+        for (int o = 0; o < 3; ++o) {
+            const int l = D == 1 ? Direction<Q>::find(ci, SIDE ? 1 : -1, o - 1) : Direction<Q>::find(ci, o - 1, SIDE ? 1 : -1);
+            if (l < Q && ok[t][o]) f1[(size_t)l * L.plane + (og + off[t][o])] = old[o];   // not ok: a halo ghost
+        }
+    }
+    if (a.halo_dir < 0 && (a.inflow_fold || per[0])) return;
+    // G - c_l beyond the face's range in a halo domain, or next to inflow planes of a separate pass.
+    // On a halo plane only: the neighbour's value of this step, pushed by that halo's unpack.  On
+    // the inflow axis only: copied above when the inflow planes are folded too, else here.  On both
+    // (the inflow ghost of a halo plane): the value that ghost holds now, the neighbour's inflow
+    // ghost from before this step.
+#pragma unroll
+    for (int l = 1; l < Q; ++l) {
+        if (Lt::c(l, D) != (SIDE ? 1 : -1)) continue;
+        int s[3] = {i, j, k};
+        bool from_inflow = false, from_halo = false;
+#pragma unroll
+        for (int t = 0; t < 2; ++t) {
+            const int d = t ? T1 : T0;
+            s[d] = x[d] - Lt::c(l, d);
+            if (per[d]) s[d] = Layout::wrap(s[d], n[d], 1);
+            else if (s[d] < 1 || s[d] > n[d]) {
+                if (d == a.halo_dir) from_halo = true;
+                else from_inflow = true;
+            }
+        }
+        if (from_inflow && (from_halo || !a.inflow_fold))
+            f1[(size_t)l * L.plane + og] = f1[(size_t)l * L.plane + L.cell(s[0], s[1], s[2])];
+    }
+}
+
 template <int Q, class C>
-__device__ __forceinline__ void fold_inflow(const StepArgs<typename C::real>& a, int i, int j, int k,
-                                            const typename C::real (&dev)[Q]) {
+__device__ __forceinline__ void fold_boundaries(const StepArgs<typename C::real>& a, int i, int j, int k, int oc,
+                                                const typename C::real (&dev)[Q]) {
     using R = typename C::real;
     using raw = typename C::raw;
     using Lt = Lattice<Q>;
     const Layout& L = a.lay;
     raw* __restrict__ f1 = static_cast<raw*>(a.dst);
-    const int gi = i == 1 ? 0 : L.nx + 1;
-    const int og = L.cell(gi, j, k);
-    const int D = a.fold_dir;
-    if (D > 0) {
-        const int x[3] = {i, j, k};
-        const int n[3] = {L.nx, L.ny, L.nz};
-        const int O = 3 - D;   // the other tangential axis: periodic or a halo axis
-        const int perO = O == 1 ? L.per_j : L.per_k;
-#pragma unroll
-        for (int side = 0; side < 2; ++side) {
-            const int plane = side ? n[D] : 1;
-            if (x[D] != plane) continue;
-#pragma unroll
-            for (int l = 0; l < Q; ++l) {
-                const int cn = Lt::c(l, D);
-                if (!(side ? cn > 0 : cn < 0)) continue;
-                // the target ghost G = (gi + c_x, x_O + c_O, ghost of D) lies in the face's range
-                if (Lt::cx(l) != (i == 1 ? 1 : -1)) continue;
-                int t[3];
-                t[0] = i;
-                t[D] = side ? n[D] + 1 : 0;
-                t[O] = x[O] + Lt::c(l, O);
-                if (perO) t[O] = Layout::wrap(t[O], n[O], 1);
-                else if (t[O] < 1 || t[O] > n[O]) continue;   // a ghost of the halo axis
-                f1[(size_t)l * L.plane + L.cell(t[0], t[1], t[2])] = f1[(size_t)l * L.plane + og];
-            }
-        }
+    const bool at_end = a.inflow_fold && (i == 1 || i == L.nx);
+    if (a.fold_dir == 0) {
+        if (i == 1) fold_face<Q, C, 0, 0>(a, i, j, k, oc, false, dev);
+        if (i == L.nx) fold_face<Q, C, 0, 1>(a, i, j, k, oc, false, dev);
+    } else if (a.fold_dir == 1) {
+        if (j == 1) fold_face<Q, C, 1, 0>(a, i, j, k, oc, at_end, dev);
+        if (j == L.ny) fold_face<Q, C, 1, 1>(a, i, j, k, oc, at_end, dev);
+    } else if (a.fold_dir == 2) {
+        if (k == 1) fold_face<Q, C, 2, 0>(a, i, j, k, oc, at_end, dev);
+        if (k == L.nz) fold_face<Q, C, 2, 1>(a, i, j, k, oc, at_end, dev);
     }
+    if (!at_end) return;
+    const int og = oc + (i == 1 ? -L.si : L.si);
     if (i == 1) {
         R fg[Q];
 #pragma unroll
@@ -740,8 +801,7 @@ __device__ __forceinline__ void step_cell(const StepArgs<typename C::real>& a, i
     }
     if (cs != ca) return;
     if (VRE && a.tau_out != nullptr) a.tau_out[occ] = tau;
-    if (a.fold_dir >= 0) fold_closed_face<Q, C>(a, i, j, k, out);
-    if (a.inflow_fold && (i == 1 || i == L.nx)) fold_inflow<Q, C>(a, i, j, k, out);
+    if (a.fold_dir >= 0 || a.inflow_fold) fold_boundaries<Q, C>(a, i, j, k, oc0, out);
 }
 
 // Threads run along the storage axes: x along the contiguous axis ax0, y along ax1, z along ax2.
@@ -817,42 +877,6 @@ template <int Q, class C>
 __device__ __forceinline__ void st(const Layout& L, void* f, int l, int off, typename C::real v) {
     static_cast<typename C::raw*>(f)[(size_t)l * (size_t)L.plane + (size_t)off] = C::template encode<Q>(v, l);
 }
-// Directions by run-time values, from packed constants (scalar shifts and masks).
-template <int Q>
-struct Outgoing {
-    // populations with c_d > 0 (side 1) or < 0 (side 0), in lattice order, five bits each
-    static constexpr int count = Q == 27 ? 9 : 5;
-    static constexpr unsigned long long pack(int d, int side) {
-        unsigned long long p = 0;
-        int n = 0;
-        for (int l = 0; l < Q; ++l)
-            if (Lattice<Q>::c(l, d) == (side ? 1 : -1)) p |= (unsigned long long)l << (5 * n++);
-        return p;
-    }
-    __device__ static __forceinline__ int pop(int d, int side, int q) {
-        constexpr unsigned long long k[6] = {pack(0, 0), pack(0, 1), pack(1, 0), pack(1, 1), pack(2, 0), pack(2, 1)};
-        const unsigned long long p = d == 0 ? (side ? k[1] : k[0]) : d == 1 ? (side ? k[3] : k[2]) : (side ? k[5] : k[4]);
-        return (int)((p >> (5 * q)) & 31ull);
-    }
-};
-template <int Q>
-struct Direction {
-    // the direction with velocity (x, y, z), 31 if the lattice has none
-    static constexpr unsigned long long pack(int part) {
-        unsigned long long p = 0;
-        for (int e = 0; e < 9; ++e) {
-            const int l = Lattice<Q>::find(part - 1, e / 3 - 1, e % 3 - 1);
-            p |= (unsigned long long)(l < 0 ? 31 : l) << (5 * e);
-        }
-        return p;
-    }
-    __device__ static __forceinline__ int find(int x, int y, int z) {
-        constexpr unsigned long long k[3] = {pack(0), pack(1), pack(2)};
-        const unsigned long long p = x < 0 ? k[0] : x == 0 ? k[1] : k[2];
-        return (int)((p >> (5 * (3 * (y + 1) + z + 1))) & 31ull);
-    }
-};
-
 // boundarycond's passes over the ghost layers of the non-periodic axes (src/m_boundarycond.F90:166-365)
 // in one launch: closed faces (src/m_boundary_{i,j,k}_closed_kernel.F90), edges and corners
 // (src/m_boundary_{j_k,i_j,i_k}_edges.F90, src/m_boundary_closed_corners.F90) and the inflow/outflow
