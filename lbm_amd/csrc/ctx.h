@@ -55,7 +55,7 @@ struct lbm_ctx {
     // actuator-line turbines (lbm_set_turbines): their forcing is written into force[] each step
     bool turb_on = false;
     lbm::TurbHost th{};
-    lbm_host::DevBuf t_rot, t_theta, t_blade, t_nfoil, t_nang, t_foil, t_pts, t_box;
+    lbm_host::DevBuf t_rot, t_theta, t_blade, t_nfoil, t_nang, t_foil, t_pts;
     // adjoint workspace (lbm_adjoint_run): checkpoints, recomputed states, adjoint buffers, the final
     // state, gradient and objective accumulators; kept between runs, grown when a run needs more
     lbm_host::DevBuf adj_ck, adj_snaps, adj_lam, adj_gF, adj_gS, adj_acc;

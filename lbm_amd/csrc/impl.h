@@ -102,7 +102,6 @@ struct TurbHost {
     const int* nang;      // [nfoils]
     const void* foil;     // [nfoils][nang_max][3]
     void* pts;            // [npts][8]
-    const int* tbox;      // [nturb][6]
     int lo[3], hi[3];     // union of the rotors' deposit boxes (i, j, k; 1-based, inclusive)
     void* F[3];           // force planes
 };

@@ -193,17 +193,16 @@ struct Launch {
             a.nang = h.nang;
             a.foil = static_cast<const R*>(h.foil);
             a.pts = static_cast<R*>(h.pts);
-            a.tbox = h.tbox;
             for (int d = 0; d < 3; ++d) {
                 a.lo[d] = h.lo[d];
                 a.hi[d] = h.hi[d];
             }
             for (int q = 0; q < 3; ++q) a.F[q] = static_cast<R*>(h.F[q]);
             hipLaunchKernelGGL((turbine_point_kernel<Q, C>), dim3(h.npts), dim3(256), 0, s, a);
-            const long long cells = (long long)(h.hi[0] - h.lo[0] + 1) * (h.hi[1] - h.lo[1] + 1) * (h.hi[2] - h.lo[2] + 1);
-            // at least one block: block 0 also stores the advanced azimuths
-            const long long blocks = cells > 0 ? (cells + 255) / 256 : 1;
-            hipLaunchKernelGGL((turbine_deposit_kernel<R>), dim3((unsigned)blocks), dim3(256), 0, s, a);
+            // at least one block: the first one also stores the advanced azimuths
+            auto ext = [&](int ax, int b) { return std::max((h.hi[ax] - h.lo[ax] + b) / b, 1); };
+            hipLaunchKernelGGL((turbine_deposit_kernel<R>), dim3(ext(L.ax0, kDepositX), ext(L.ax1, kDepositY), ext(L.ax2, 1)),
+                               dim3(kDepositX * kDepositY), 0, s, a);
             return hipGetLastError();
         }
     }

@@ -65,14 +65,13 @@ int lbm_set_turbines(lbm_ctx* c, const lbm_turbines* t) {
     const int n[3] = {d.nx, d.ny, d.nz};
     auto R = [&](double v) { return round_real(c, v); };
     // Rotor table: hub, rotor basis (src/m_turbine_rotor_basis.F90:19-21, evaluated once here in the
-    // compute precision), omegand, pitch.  Deposit box of each rotor: every point lies within
+    // compute precision), omegand, pitch.  Deposit box, the union over the rotors: every point lies within
     // relm_max * |(e1_d, e2_d)| of the hub along axis d; its stencil reaches krad cells beyond.
     const double sigma = R(R(2.0) / R(std::sqrt(R(2.0))));
     const int krad = std::min(5, (int)std::ceil(R(R(3.0) * sigma)));   // src/m_turbine_deposit.F90:36-38
     double relm_max = 0;
     for (int q = 0; q < t->nchords; ++q) relm_max = std::max(relm_max, std::fabs(R(t->relm[q])));
     std::vector<double> rot((size_t)t->nturbines * kTurbRot, 0.0);
-    std::vector<int> box((size_t)t->nturbines * 6);
     int lo[3] = {n[0], n[1], n[2]}, hi[3] = {1, 1, 1};
     for (int m = 0; m < t->nturbines; ++m) {
         double* r = &rot[(size_t)m * kTurbRot];
@@ -94,8 +93,6 @@ int lbm_set_turbines(lbm_ctx* c, const lbm_turbines* t) {
             const double reach = relm_max * std::sqrt(e1[a] * e1[a] + e2[a] * e2[a]);
             const int blo = std::max(1, (int)std::floor(r[a] - reach) - krad - 1);
             const int bhi = std::min(n[a], (int)std::floor(r[a] + reach) + krad + 1);
-            box[6 * m + 2 * a] = blo;
-            box[6 * m + 2 * a + 1] = bhi;
             lo[a] = std::min(lo[a], blo);
             hi[a] = std::max(hi[a], bhi);
         }
@@ -121,7 +118,6 @@ int lbm_set_turbines(lbm_ctx* c, const lbm_turbines* t) {
         (rc = upload(c, c->t_foil, img_foil.data(), img_foil.size())) ||
         (rc = upload(c, c->t_nfoil, nfoil.data(), nfoil.size() * sizeof(int))) ||
         (rc = upload(c, c->t_nang, nang.data(), nang.size() * sizeof(int))) ||
-        (rc = upload(c, c->t_box, box.data(), box.size() * sizeof(int))) ||
         (rc = dev_alloc(c, c->t_pts, (size_t)npts * kTurbPt * rb)))
         return rc;
     // force planes: zero outside the deposit box, which the deposit rewrites every step
@@ -146,7 +142,6 @@ int lbm_set_turbines(lbm_ctx* c, const lbm_turbines* t) {
     h.nang = static_cast<const int*>(c->t_nang.p);
     h.foil = c->t_foil.p;
     h.pts = c->t_pts.p;
-    h.tbox = static_cast<const int*>(c->t_box.p);
     for (int a = 0; a < 3; ++a) {
         h.lo[a] = lo[a];
         h.hi[a] = hi[a];
