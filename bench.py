@@ -18,7 +18,7 @@ Prints ONE JSON line.  --gpus N > 1 is refused: this build targets one GPU.
 
 times the batched ensemble instead: 64 D3Q19 regularized + Vreman members with sizes drawn by
 seed from {96,128,160}x{64,96}x{64,96}, a seeded box obstacle (side 8-16) and seeded inflow
-forcing each, FP32, graph-captured batched steps with the autotuned launch shape, against the
+forcing each, FP32, batched steps with the autotuned launch shape, against the
 same members stepped with one launch sequence per member; --small-members draws the sizes from
 {24,32,40}x{16,24}x{16,24} (box side 4-8) instead.
 
@@ -222,7 +222,7 @@ def bench_ensemble(a):
                      # measured for the default ensemble (64 FP32 members) only
                      "traffic": (traffic_from_profiles("ensemble_step_kernel_batch_q19_64members")
                                  if a.storage == "f32" and a.members == 64 and not a.small_members else None),
-                     "kernel": "step_kernel_batch (graph; faces and inflow planes folded)", "bytes_per_cell": bpc_bytes,
+                     "kernel": "step_kernel_batch (faces and inflow planes folded)", "bytes_per_cell": bpc_bytes,
                      "kernel_ms": round(step_ms, 5)},
         "tuned_launch": {"block": block, "blocks_per_cu": bpc, "ms_per_step": round(tune_ms, 5)},
         "per_member_launches": {"value": round(mlups_pm, 1), "unit": "MLUPS", "steps": n_pm,

@@ -267,9 +267,8 @@ int lbm_get_info(lbm_ctx* ctx, int64_t* device_bytes, int32_t* row_pitch, int64_
 /*
  * Ensembles.  No counterpart in the reference, which runs one domain per process: many contexts
  * of one lattice, storage and collision model (sizes, boundary codes, solids, inflow and
- * turbulence inputs free per member) advance together.  Each step is one launch of a persistent
- * batched step kernel over every member's cells, one launch of a batched inflow/outflow kernel
- * and a device clock tick, captured in HIP graphs.  Members keep behaving as their own contexts:
+ * turbulence inputs free per member) advance together.  Each step is one launch of a batched step
+ * kernel over every member's cells.  Members keep behaving as their own contexts:
  * lbm_get_state / lbm_get_macros / lbm_set_* on a member work between ensemble steps (a member
  * changed with lbm_set_* is picked up by the next lbm_ensemble_step), and the result is exactly
  * that of lbm_step on each member.  A member may have at most one closed (11/12/21/22) axis,

@@ -1,13 +1,12 @@
 // Ensembles (lbm_ensemble_* in include/lbm_hip.h): many single-domain contexts advanced together
-// by one launch of the batched step kernel per step, with the step sequence captured in HIP
-// graphs and the launch shape chosen by a measuring autotuner.  The reference runs one domain
+// by one launch of the batched step kernel per step, with the launch shape chosen by a measuring
+// autotuner.  The reference runs one domain
 // per process; each member here behaves exactly as lbm_step on its own context would (same
 // kernels, same arithmetic), which is what the tests check.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
 #include <cstring>
-#include <map>
 #include <string>
 #include <vector>
 
@@ -19,7 +18,6 @@ using namespace lbm;
 using namespace lbm_host;
 
 namespace {
-constexpr int kGraphSteps = 16;    // steps per captured graph
 constexpr int kChunk = 1024;       // steps per upload of the per-step inflow values
 }  // namespace
 
@@ -36,14 +34,10 @@ struct lbm_ens {
     int block = 256;
     int bpc = 0;                   // persistent grid of bpc blocks per CU; 0: one block per tile
     // device tables and their host images
-    DevBuf tab, owner, vals, clock, backup;
+    DevBuf tab, owner, vals, backup;
     std::vector<unsigned char> h_tab, h_vals;
     std::vector<int> h_owner;
-    int h_clock[3] = {0, 0, 0};
     EnsLaunch L{};
-    // captured graphs by number of steps, valid for the launch in `key`
-    std::map<int, hipGraphExec_t> graphs;
-    std::vector<long long> key;
     // timing
     bool timing = false;
     std::vector<hipEvent_t> ev;
@@ -88,16 +82,11 @@ int ealloc(lbm_ens* e, DevBuf& b, size_t n, bool* moved) {
     return LBM_OK;
 }
 
-void drop_graphs(lbm_ens* e) {
-    for (auto& g : e->graphs) hipGraphExecDestroy(g.second);
-    e->graphs.clear();
-}
-
 int closed_axes(const lbm_desc& d) {
     return (d.ibnd > 10) + (d.jbnd > 10) + (d.kbnd > 10);
 }
 
-// Member tables for the current launch shape; drops the graphs when a kernel argument changes.
+// Member tables for the current launch shape.
 int build_tables(lbm_ens* e) {
     const int n = (int)e->mem.size();
     const size_t mb = e->ops->member_bytes;
@@ -125,10 +114,9 @@ int build_tables(lbm_ens* e) {
         own.resize((size_t)total, m);
     }
     bool moved = false;
-    if (int rc = ealloc(e, e->tab, mb * n, &moved)) return rc;
+    if (int rc = ealloc(e, e->tab, mb * n, nullptr)) return rc;
     if (int rc = ealloc(e, e->owner, sizeof(int) * own.size(), &moved)) return rc;
-    if (int rc = ealloc(e, e->clock, sizeof(e->h_clock), &moved)) return rc;
-    if (int rc = ealloc(e, e->vals, (size_t)kChunk * n * 3 * e->ops->real_bytes, &moved)) return rc;
+    if (int rc = ealloc(e, e->vals, (size_t)kChunk * n * 3 * e->ops->real_bytes, nullptr)) return rc;
     EHIP(e, hipMemcpyAsync(e->tab.p, e->h_tab.data(), mb * n, hipMemcpyHostToDevice, e->stream));
     if (moved || own != e->h_owner) {
         e->h_owner.swap(own);
@@ -137,47 +125,12 @@ int build_tables(lbm_ens* e) {
     EnsLaunch& L = e->L;
     L.tab = e->tab.p;
     L.owner = static_cast<const int*>(e->owner.p);
-    L.nmem = n;
     L.total = (int)total;
     L.block = e->block;
     L.grid = e->bpc > 0 ? (int)std::min<long long>(total, (long long)e->bpc * e->cus) : (int)total;
-    L.vals = e->vals.p;
-    L.clock = static_cast<int*>(e->clock.p);
     L.bgk3 = e->bgk3;
     L.hrr = e->hrr;
     L.vre = e->vre;
-    std::vector<long long> key = {(long long)(size_t)L.tab, (long long)(size_t)L.owner, L.nmem, L.total, L.block,
-                                  L.grid, (long long)(size_t)L.vals, (long long)(size_t)L.clock};
-    if (moved || key != e->key) {
-        drop_graphs(e);
-        e->key = key;
-    }
-    return LBM_OK;
-}
-
-int graph_for(lbm_ens* e, int steps, hipGraphExec_t* out) {
-    auto it = e->graphs.find(steps);
-    if (it != e->graphs.end()) {
-        *out = it->second;
-        return LBM_OK;
-    }
-    EHIP(e, hipStreamBeginCapture(e->stream, hipStreamCaptureModeThreadLocal));
-    hipError_t le = hipSuccess;
-    for (int s = 0; s < steps && le == hipSuccess; ++s) le = e->ops->ens_step(e->L, s, e->stream);
-    if (le == hipSuccess) le = e->ops->ens_tick(e->L, steps, e->stream);
-    hipGraph_t g = nullptr;
-    const hipError_t ce = hipStreamEndCapture(e->stream, &g);
-    if (le != hipSuccess) {
-        if (g) hipGraphDestroy(g);
-        return efail(e, LBM_EHIP, std::string("batched step launch: ") + hipGetErrorString(le));
-    }
-    if (ce != hipSuccess) return efail(e, LBM_EHIP, std::string("hipStreamEndCapture: ") + hipGetErrorString(ce));
-    hipGraphExec_t x = nullptr;
-    const hipError_t ie = hipGraphInstantiate(&x, g, nullptr, nullptr, 0);
-    hipGraphDestroy(g);
-    if (ie != hipSuccess) return efail(e, LBM_EHIP, std::string("hipGraphInstantiate: ") + hipGetErrorString(ie));
-    e->graphs[steps] = x;
-    *out = x;
     return LBM_OK;
 }
 
@@ -213,20 +166,11 @@ int batched(lbm_ens* e, int it0, int nsteps) {
                 }
             }
         EHIP(e, hipMemcpyAsync(e->vals.p, e->h_vals.data(), e->h_vals.size(), hipMemcpyHostToDevice, e->stream));
-        e->h_clock[0] = it0 + done + 1;
-        e->h_clock[1] = done;   // buffer parity: steps since the members' current buffers were taken
-        e->h_clock[2] = done;   // the uploaded table's first step
-        EHIP(e, hipMemcpyAsync(e->clock.p, e->h_clock, sizeof(e->h_clock), hipMemcpyHostToDevice, e->stream));
         hipEvent_t t0 = nullptr;
         if (e->timing && (t0 = next_ev(e))) hipEventRecord(t0, e->stream);
-        int left = chunk;
-        while (left > 0) {
-            const int g = std::min(left, kGraphSteps);
-            hipGraphExec_t x;
-            if (int rc = graph_for(e, g, &x)) return rc;
-            EHIP(e, hipGraphLaunch(x, e->stream));
-            left -= g;
-        }
+        for (int q = 0; q < chunk; ++q)
+            EHIP(e, e->ops->ens_step(e->L, it0 + done + q + 1, done + q,
+                                     static_cast<const char*>(e->vals.p) + (size_t)q * n * 3 * rb, e->stream));
         if (e->timing && t0) {
             hipEvent_t t1 = next_ev(e);
             if (t1) hipEventRecord(t1, e->stream);
@@ -307,8 +251,7 @@ int lbm_ensemble_destroy(lbm_ens* e) {
     if (int rc = check_ens(e)) return rc;
     e->tag = 0;
     if (e->stream) hipStreamSynchronize(e->stream);
-    drop_graphs(e);
-    for (DevBuf* b : {&e->tab, &e->owner, &e->vals, &e->clock, &e->backup}) dev_free(*b);
+    for (DevBuf* b : {&e->tab, &e->owner, &e->vals, &e->backup}) dev_free(*b);
     for (hipEvent_t x : e->ev) hipEventDestroy(x);
     for (hipEvent_t x : e->ev_mem)
         if (x) hipEventDestroy(x);
@@ -456,7 +399,7 @@ int lbm_ensemble_tune(lbm_ens* e, int it0, int trial_steps, int* best_block, int
             e->block = b;
             e->bpc = p;
             e->timing = false;
-            if ((rc = lbm_ensemble_step(e, it0, 2))) break;            // first step, graph capture
+            if ((rc = lbm_ensemble_step(e, it0, 2))) break;            // first step, warm-up
             if (hipEventRecord(t0, e->stream) != hipSuccess) { rc = efail(e, LBM_EHIP, "hipEventRecord"); break; }
             if ((rc = lbm_ensemble_step(e, it0 + 2, trial_steps))) break;
             if (hipEventRecord(t1, e->stream) != hipSuccess || hipEventSynchronize(t1) != hipSuccess) {

@@ -83,9 +83,7 @@ struct MemberHost {
 struct EnsLaunch {
     const void* tab;                 // device MemberTab<R>[nmem]
     const int* owner;                // device member of each tile [total]
-    int nmem, total, block, grid;
-    const void* vals;                // device (utime, cos, sin)[steps of the table][nmem]
-    int* clock;                      // device {it of a graph's first step, steps since set, table's first step}
+    int total, block, grid;
     int bgk3, hrr, vre;
 };
 
@@ -148,8 +146,8 @@ struct Ops {
     // ensembles
     size_t member_bytes;   // sizeof(MemberTab<R>)
     void (*ens_pack)(const MemberHost&, int block, int start, void* out, long long* tiles);
-    hipError_t (*ens_step)(const EnsLaunch&, int sub, hipStream_t);   // step clock + sub
-    hipError_t (*ens_tick)(const EnsLaunch&, int steps, hipStream_t);
+    // step it, done steps after the member tables were made; vals: device (utime, cos, sin)[nmem] of it
+    hipError_t (*ens_step)(const EnsLaunch&, int it, int done, const void* vals, hipStream_t);
     // adjoint (nullptr for the 16-bit storage codecs)
     hipError_t (*adj_step)(const Layout&, const StepHost&, const void* lam_y, void* lam_x, const AdjBox&, double kappa,
                            int coll, double* gF, hipStream_t);

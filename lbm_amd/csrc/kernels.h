@@ -1201,21 +1201,20 @@ __global__ void __launch_bounds__(256) halo_unpack_kernel(Layout L, void* f, int
 // consecutive cells, which the first form cut regardless of rows, left lines of rows that are no
 // multiple of 64 cells to two waves, whose separate partial stores memory read and wrote twice.
 // Measured on MI355X, D3Q19 per step: 16 members of about 112x84x70 cells (10.8 M) FP32 560 -> 319 us,
-// FP64 880 -> 641 us, FP16 388 -> 242 us; 64 of about 28x21x17 (0.61 M) FP32 59 -> 46 us, of it 10 us
-// for the clock's launch; 16 members of 96-160x64-96x64-96 (14.2 M), most rows aligned before, 402 ->
+// FP64 880 -> 641 us, FP16 388 -> 242 us; 64 of about 28x21x17 (0.61 M) FP32 59 -> 46 us; 16 members of 96-160x64-96x64-96 (14.2 M), most rows aligned before, 402 ->
 // 386 us.
 //
-// Per-step values are read from a device clock (clock[0] = it of the first step of a captured graph,
-// clock[1] = steps done since the clock was set, clock[2] = the value of clock[1] at the first step of
-// the uploaded table of inflow values), to which each launch adds its place sub in the graph; the
-// graph's end advances the clock, so that it replays without host updates.  Each member's closed face and inflow/outflow planes are
-// folded into the step (at most one closed axis per member).
+// A step is one plain launch, with the step number and the buffers' parity as arguments.  Captured in
+// graphs of 16 steps, which had to read them from a device clock, the steps were further apart than
+// launches queued on a stream: 64 small members FP32 46.3 -> 42.9 us per step, FP16 44.4 -> 39.9 us, 16
+// ordinary ones FP16 242 -> 232 us, FP32 and FP64 as before.  Each member's closed face and inflow/outflow planes are folded into the
+// step (at most one closed axis per member).
 // ------------------------------------------------------------------------------------------
 template <typename R>
 struct MemberTab {
     StepArgs<R> a;          // src, dst, tu, tv, tw are set per step
     void* buf[2];
-    int cur0;               // buffer holding the current state when the clock was set
+    int cur0;               // buffer holding the current state when the table was made
     int nrturb, slice;      // turbulence slices of ny*nz reals; nrturb = 0: off
     const R* turb[3];       // slice 0 of uu, vv, ww
     int seg_row, tiles_plane;   // segments per row; tiles per (ax0, ax1) plane
@@ -1226,18 +1225,14 @@ struct MemberTab {
 template <typename raw>
 constexpr int kSegment = 64 / (int)sizeof(raw);
 
-// vals: (uvel_time(it), cos(udir), sin(udir)) per step of the table and member; owner: the member of
-// each tile.
+// it: the step; s: steps done since the table was made; vals: the step's (uvel_time(it), cos(udir),
+// sin(udir)) per member; owner: the member of each tile.
 template <int Q, class C, bool BGK3, bool HRR, bool VRE>
 __global__ void __launch_bounds__(1024) step_kernel_batch(const MemberTab<typename C::real>* __restrict__ tab,
-                                                          const int* __restrict__ owner, int nmem, int total,
-                                                          const typename C::real* __restrict__ vals,
-                                                          const int* __restrict__ clock, int sub) {
+                                                          const int* __restrict__ owner, int total, int it, int s,
+                                                          const typename C::real* __restrict__ vals) {
     using R = typename C::real;
     constexpr unsigned W = kSegment<typename C::raw>;
-    const int it = clock[0] + sub;
-    const int s = clock[1] + sub;
-    const int sv = s - clock[2];
     for (int t = blockIdx.x; t < total; t += gridDim.x) {
         const int m = owner[t];
         const MemberTab<R>& M = tab[m];
@@ -1246,7 +1241,7 @@ __global__ void __launch_bounds__(1024) step_kernel_batch(const MemberTab<typena
         a.src = M.buf[p];
         a.dst = M.buf[p ^ 1];
         if (a.inflow_fold) {
-            const R* v = vals + ((size_t)sv * nmem + m) * 3;
+            const R* v = vals + (size_t)m * 3;
             a.utime = v[0];
             a.cosd = v[1];
             a.sind = v[2];
@@ -1265,14 +1260,6 @@ __global__ void __launch_bounds__(1024) step_kernel_batch(const MemberTab<typena
         const unsigned u = e / W;
         const unsigned cb = u / (unsigned)M.seg_row;
         step_cell<Q, C, BGK3, HRR, VRE, 1>(a, (int)((u - cb * (unsigned)M.seg_row) * W + e % W) + 1, (int)cb + 1, cc + 1);
-    }
-}
-
-template <int Q, class C>
-__global__ void clock_tick_kernel(int* clock, int steps) {
-    if (threadIdx.x == 0) {
-        clock[0] += steps;
-        clock[1] += steps;
     }
 }
 

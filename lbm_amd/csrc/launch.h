@@ -346,30 +346,25 @@ struct Launch {
     }
 
     template <bool B3, bool H, bool V>
-    static void ens_step_t(const EnsLaunch& e, int sub, hipStream_t s) {
+    static void ens_step_t(const EnsLaunch& e, int it, int done, const void* vals, hipStream_t s) {
         if constexpr (kNT)
             hipLaunchKernelGGL((step_kernel_batch<Q, C, B3, H, V>), dim3(e.grid), dim3(e.block), 0, s,
-                               static_cast<const MemberTab<R>*>(e.tab), e.owner, e.nmem, e.total,
-                               static_cast<const R*>(e.vals), e.clock, sub);
+                               static_cast<const MemberTab<R>*>(e.tab), e.owner, e.total, it, done,
+                               static_cast<const R*>(vals));
     }
 
-    static hipError_t ens_step(const EnsLaunch& e, int sub, hipStream_t s) {
+    static hipError_t ens_step(const EnsLaunch& e, int it, int done, const void* vals, hipStream_t s) {
         const int key = (e.bgk3 ? 4 : 0) | (e.hrr ? 2 : 0) | (e.vre ? 1 : 0);
         switch (key) {
-            case 0: ens_step_t<false, false, false>(e, sub, s); break;
-            case 1: ens_step_t<false, false, true>(e, sub, s); break;
-            case 2: ens_step_t<false, true, false>(e, sub, s); break;
-            case 3: ens_step_t<false, true, true>(e, sub, s); break;
-            case 4: ens_step_t<true, false, false>(e, sub, s); break;
-            case 5: ens_step_t<true, false, true>(e, sub, s); break;
-            case 6: ens_step_t<true, true, false>(e, sub, s); break;
-            default: ens_step_t<true, true, true>(e, sub, s); break;
+            case 0: ens_step_t<false, false, false>(e, it, done, vals, s); break;
+            case 1: ens_step_t<false, false, true>(e, it, done, vals, s); break;
+            case 2: ens_step_t<false, true, false>(e, it, done, vals, s); break;
+            case 3: ens_step_t<false, true, true>(e, it, done, vals, s); break;
+            case 4: ens_step_t<true, false, false>(e, it, done, vals, s); break;
+            case 5: ens_step_t<true, false, true>(e, it, done, vals, s); break;
+            case 6: ens_step_t<true, true, false>(e, it, done, vals, s); break;
+            default: ens_step_t<true, true, true>(e, it, done, vals, s); break;
         }
-        return hipGetLastError();
-    }
-
-    static hipError_t ens_tick(const EnsLaunch& e, int steps, hipStream_t s) {
-        hipLaunchKernelGGL((clock_tick_kernel<Q, C>), dim3(1), dim3(64), 0, s, e.clock, steps);
         return hipGetLastError();
     }
 
@@ -445,7 +440,7 @@ struct Launch {
     static const Ops* ops() {
         static const Ops o = {&step, &boundary, &aos_in, &state_out, &moments_out,
                               &averages_out, &field_in, &feq_init, &totals, &average,
-                              sizeof(MemberTab<R>), &ens_pack, &ens_step, &ens_tick,
+                              sizeof(MemberTab<R>), &ens_pack, &ens_step,
                               kAdj ? &adj_step : nullptr, kAdj ? &adj_inflow : nullptr, kAdj ? &adj_face : nullptr,
                               &objective, &halo_pack, &halo_unpack, &ghost_copy, &turb_step, (int)sizeof(R),
                               (int)sizeof(typename C::raw)};
