@@ -161,27 +161,36 @@ __global__ void __launch_bounds__(256) turbine_point_kernel(const TurbArgs<typen
     const int kf = a.nfoil[c];
     const int rows = a.nang[kf];
     const R* tab = a.foil + (size_t)kf * a.nang_max * 3;
-    R dens = 0, ux = 0, utheta = 0, phi = 0;
-    if (tid == 0) {
-        dens = turbine_trilinear(corner[0], fr[0], fr[1], fr[2]);
-        ux = turbine_trilinear(corner[1], fr[0], fr[1], fr[2]);
+    // src/m_turbine_point_forces_kernel.F90:57-66
+    struct Flow {
+        R dens, ux, utheta, phi, ang;
+    };
+    auto flow = [&]() {
+        Flow f;
+        f.dens = turbine_trilinear(corner[0], fr[0], fr[1], fr[2]);
+        f.ux = turbine_trilinear(corner[1], fr[0], fr[1], fr[2]);
         const R uy = turbine_trilinear(corner[2], fr[0], fr[1], fr[2]);
         const R uz = turbine_trilinear(corner[3], fr[0], fr[1], fr[2]);
-        // src/m_turbine_point_forces_kernel.F90:57-66
-        utheta = omegand * relm - uz * ct - uy * st;
-        phi = t_atan2(ux, utheta);
-        s_ang = phi * R(180) / pi - bl[3] - rot[13];
+        f.utheta = omegand * relm - uz * ct - uy * st;
+        f.phi = t_atan2(f.ux, f.utheta);
+        f.ang = f.phi * R(180) / pi - bl[3] - rot[13];
+        return f;
+    };
+    if (tid == 0) {
+        s_ang = flow().ang;
         s_row = rows;
     }
     __syncthreads();
     // src/m_nrelliftdrag.F90:17-33: linear in the first interval deg(i) < ang <= deg(i+1); the whole
     // table is looked at at once (one thread going down its rows, a load at a time, took the kernel from
     // 8.5 to 14.6 us)
-    const R ang = s_ang;
     for (int i = tid; i + 1 < rows; i += blockDim.x)
-        if (tab[3 * i] < ang && ang <= tab[3 * i + 3]) atomicMin(&s_row, i);
+        if (tab[3 * i] < s_ang && s_ang <= tab[3 * i + 3]) atomicMin(&s_row, i);
     __syncthreads();
     if (tid != 0) return;
+    // (again, so that the force's expressions are compiled as a whole and round as they did)
+    const Flow fl = flow();
+    const R dens = fl.dens, ux = fl.ux, utheta = fl.utheta, phi = fl.phi, ang = fl.ang;
     R clift = 0, cdrag = 0;
     const int i = s_row;
     if (i + 1 < rows) {
