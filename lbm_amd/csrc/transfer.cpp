@@ -12,11 +12,12 @@
 
 #include <algorithm>
 #include <atomic>
+#include <condition_variable>
 #include <cstring>
+#include <exception>
+#include <memory>
 #include <mutex>
-#include <system_error>
 #include <thread>
-#include <vector>
 
 namespace lbm_host {
 
@@ -39,6 +40,11 @@ struct Job {
     size_t total, chunks;
     std::atomic<size_t> next{0};
     std::atomic<int> error{hipSuccess};
+    // threads that take part; none joins any more once the calling thread has run out of chunks
+    std::mutex mu;
+    std::condition_variable idle;
+    int active = 0;
+    bool closed = false;
 };
 
 // Everything of the device range's chunk k that a part holds or wants, from or to the slot.
@@ -100,8 +106,23 @@ void work(Job& j, int w) {
         if (e) (void)hipEventDestroy(e);
 }
 
+// A thread of the team.  One that the system starts late (other threads of the process may keep all
+// processors busy) finds the job closed, and nobody waits for it: joined threads made copies of 16 MB
+// slower than the runtime's beside a spinning OpenMP team.
+void join_in(std::shared_ptr<Job> j, int w) {
+    {
+        std::lock_guard<std::mutex> lk(j->mu);
+        if (j->closed) return;
+        ++j->active;
+    }
+    work(*j, w);
+    std::lock_guard<std::mutex> lk(j->mu);
+    if (--j->active == 0) j->idle.notify_all();
+}
+
 int copy(lbm_ctx* c, char* dev, const HostPart* parts, int n, bool in) {
-    Job j;
+    const std::shared_ptr<Job> job = std::make_shared<Job>();
+    Job& j = *job;
     j.c = c;
     j.dev = dev;
     j.parts = parts;
@@ -137,15 +158,17 @@ int copy(lbm_ctx* c, char* dev, const HostPart* parts, int n, bool in) {
     }
     // a thread costs about as much as emptying a slot: one for every two chunks
     const int threads = (int)std::min<size_t>(kWorkers, (j.chunks + 1) / 2);
-    std::vector<std::thread> team;
     try {
-        team.reserve(threads - 1);
-        for (int w = 1; w < threads; ++w) team.emplace_back(work, std::ref(j), w);
+        for (int w = 1; w < threads; ++w) std::thread(join_in, job, w).detach();
     } catch (const std::exception&) {
         // fewer threads than wanted: the others take their chunks
     }
     work(j, 0);
-    for (std::thread& t : team) t.join();
+    {
+        std::unique_lock<std::mutex> lk(j.mu);
+        j.closed = true;
+        j.idle.wait(lk, [&] { return j.active == 0; });
+    }
     if (j.error.load() != hipSuccess) {
         (void)hipStreamSynchronize(c->stream);   // nothing still uses the slots
         return hipfail(c, (hipError_t)j.error.load(), in ? "copy to the device" : "copy to the host");
