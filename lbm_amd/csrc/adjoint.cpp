@@ -2,7 +2,7 @@
 // No counterpart in the reference: they differentiate its time loop.
 //
 // The adjoint run advances the context nsteps steps from its current state, storing every `every`
-// steps a checkpoint (the state and the ghost shell of the state before it).  The reverse sweep
+// steps a checkpoint (the state and the ghosts of the state before it that a step keeps).  The reverse sweep
 // walks the segments from last to first: it recomputes the segment's states from its checkpoint
 // (kept as full buffers, ghosts included: they are the inputs of the steps to reverse) and reverses
 // the steps with the kernels of adjoint.h.  The sweep leaves the context's buffers alone, so the
@@ -164,7 +164,7 @@ int lbm_adjoint_run(lbm_ctx* c, int it0, int nsteps, int every, const int32_t* b
     };
     int rc = LBM_OK;
     const bool want_gF = grad_force && c->has_force;
-    // a checkpoint: X(n0) and the ghost shell of X(n0-1); the segment's states X(n0+1) .. X(n1-1) in
+    // a checkpoint: X(n0) and the kept ghosts of X(n0-1); the segment's states X(n0+1) .. X(n1-1) in
     // `every - 1` slots (X(n0) is read from the checkpoint)
     if ((rc = dev_alloc(c, ck, (size_t)nck * 2 * bb)) || (rc = dev_alloc(c, snaps, (size_t)std::max(every - 1, 1) * bb)) ||
         (rc = dev_alloc(c, lam, 2 * bb)) ||
@@ -179,6 +179,13 @@ int lbm_adjoint_run(lbm_ctx* c, int it0, int nsteps, int every, const int32_t* b
     char* snp = static_cast<char*>(snaps.p);
     char* lmp = static_cast<char*>(lam.p);
     std::vector<int> ck_cur(nck, 0);
+    // what a step into `to` needs of the state before the last (ghost_keep_kernel): nothing unless inflow
+    // planes meet a closed axis
+    auto ghosts = [&](const void* from, void* to) -> int {
+        if (d.ibnd != 1 || c->fold_dir < 0) return LBM_OK;
+        HIPCHK(c, c->ops->ghost_keep(c->lay, from, to, c->fold_dir, c->stream));
+        return LBM_OK;
+    };
     auto run = [&]() -> int {
         const int nblk = objective_blocks(b);
         HIPCHK(c, hipMemsetAsync(acc.p, 0, 2 * (size_t)nblk * sizeof(double), c->stream));
@@ -188,7 +195,7 @@ int lbm_adjoint_run(lbm_ctx* c, int it0, int nsteps, int every, const int32_t* b
                 const int q = (n - 1) / every;
                 ck_cur[q] = c->cur;   // the ping-pong parity of X(n0), which the adjoint buffers follow
                 if (int r = copy_dev(c, ckp + (size_t)q * 2 * bb, c->buf[c->cur], bb)) return r;
-                HIPCHK(c, c->ops->ghost_copy(c->lay, c->buf[c->cur ^ 1], ckp + (size_t)q * 2 * bb + bb, c->stream));
+                if (int r = ghosts(c->buf[c->cur ^ 1], ckp + (size_t)q * 2 * bb + bb)) return r;
             }
             if (int r = lbm_step(c, it0 + n - 1, 1)) return r;
             HIPCHK(c, c->ops->objective(c->lay, c->buf[c->cur], b, static_cast<double*>(acc.p), c->stream));
@@ -219,8 +226,8 @@ int lbm_adjoint_run(lbm_ctx* c, int it0, int nsteps, int every, const int32_t* b
             const int n0 = seg * every, n1 = std::min(n0 + every, nsteps);
             // the inputs X(n0) .. X(n1-1) of the segment's steps, slot m holding X(n0+m): slot 0 is
             // the checkpoint's X(n0) (read in place); step n0+m is written straight into slot m after
-            // that slot received the ghost shell of X(n0+m-2) (slot m-2, or the checkpoint's shell of
-            // X(n0-1)), which is what the buffer receiving that step holds in the forward run's
+            // that slot received the kept ghosts of X(n0+m-2) (slot m-2, or the checkpoint's of X(n0-1)),
+            // which is what the buffer receiving that step holds in the forward run's
             // ping-pong
             char* ckx = ckp + (size_t)seg * 2 * bb;
             char* x_before = ckx + bb;
@@ -228,7 +235,7 @@ int lbm_adjoint_run(lbm_ctx* c, int it0, int nsteps, int every, const int32_t* b
             for (int n = n0 + 1; n < n1; ++n) {
                 const int m = n - n0;
                 char* dst = slot(m);
-                HIPCHK(c, c->ops->ghost_copy(c->lay, m >= 2 ? slot(m - 2) : x_before, dst, c->stream));
+                if (int r = ghosts(m >= 2 ? slot(m - 2) : x_before, dst)) return r;
                 if (int r = step_buffers(c, slot(m - 1), dst, it0 + n)) return r;
             }
             for (int n = n1; n > n0; --n) {

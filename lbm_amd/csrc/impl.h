@@ -158,7 +158,9 @@ struct Ops {
     // halo planes of j (side 0: j = 1 / ghost 0, side 1: j = ny / ghost ny+1)
     hipError_t (*halo_pack)(const Layout&, const void* f, int side, void* buf, hipStream_t);
     hipError_t (*halo_unpack)(const Layout&, void* f, int side, const void* buf, int fold_dir, hipStream_t);
-    hipError_t (*ghost_copy)(const Layout&, const void* src, void* dst, hipStream_t);
+    // ghosts at the inflow planes of i and the closed axis D (1 or 2) that a step leaves or reads before
+    // it writes them
+    hipError_t (*ghost_keep)(const Layout&, const void* src, void* dst, int D, hipStream_t);
     // turbine forcing of one step from the step's input (src, stream as the step kernel's; ext: the
     // moments of an equilibrium start or nullptr)
     hipError_t (*turb_step)(const Layout&, const TurbHost&, const void* src, int stream, const void* const ext[4],

@@ -1055,45 +1055,30 @@ __global__ void __launch_bounds__(256) boundary_kernel(const BoundaryArgs<typena
     f1[at(l, g)] = along;
 }
 
-// Ghost shell of a buffer (the ghost cells of the non-periodic axes, all populations; periodic
-// axes' ghosts are never read) copied from src to dst: a buffer about to receive a step's output
-// then holds the ghosts it would hold had it received the step before it (the adjoint's recompute
-// writes each step into a snapshot slot of its own instead of ping-ponging two buffers).
-// Work items in storage coordinates (a, b, c) along (ax0, ax1, ax2): blocks [0, nr1) copy the rows
-// b = 0, n1+1 (every c), blocks [nr1, nr1 + nr2) the rows c = 0, n2+1 (interior b), the remaining
-// blocks the two end cells a = 0, n0+1 of the interior rows; nr1, nr2, the end cells are zero for a
-// periodic axis.
+// The ghosts that a step needs its output buffer to hold beforehand, copied from src to dst: dst then
+// receives the step as if it had received the one before the last (the adjoint's recompute writes each
+// step into a snapshot slot of its own instead of ping-ponging two buffers).  With at most one closed axis
+// D a step rewrites every ghost that anything reads but two kinds, both at an inflow plane of i next to a
+// closed D (j or k), which is where the kernel copies: the edges (D = 0, n + 1), which no pass writes, and the
+// wall planes (D = 1, n), whose values from before the step the face pass reads.  (Populations that
+// move along a closed face are neither written nor read in its ghosts.)  One thread per value, along the
+// periodic axis T.  Copying the whole shell, a thread per ghost cell, took 11.4 us of a D3Q19 FP32 step
+// of 192x96x96 cells; this takes 4.8 us.
 template <int Q, class C>
-__global__ void __launch_bounds__(256) ghost_copy_kernel(Layout L, const void* src, void* dst, int nr1, int nr2) {
+__global__ void __launch_bounds__(256) ghost_keep_kernel(Layout L, const void* src, void* dst, int D) {
     using raw = typename C::raw;
-    const int n0 = L.n(L.ax0), n1 = L.n(L.ax1), n2 = L.n(L.ax2);
-    const raw* __restrict__ s = static_cast<const raw*>(src);
-    raw* __restrict__ d = static_cast<raw*>(dst);
-    auto copy = [&](int a, int b, int c) {
-        int i, j, k;
-        L.ijk(a, b, c, i, j, k);
-        const int o = L.cell(i, j, k);
-#pragma unroll
-        for (int l = 0; l < Q; ++l) d[(size_t)l * L.plane + o] = s[(size_t)l * L.plane + o];
-    };
-    const int r = blockIdx.x;
-    if (r < nr1 + nr2) {
-        int b, c;
-        if (r < nr1) {
-            b = (r & 1) ? n1 + 1 : 0;
-            c = r >> 1;
-        } else {
-            const int r2 = r - nr1;
-            c = (r2 & 1) ? n2 + 1 : 0;
-            b = (r2 >> 1) + 1;
-        }
-        for (int a = threadIdx.x; a <= n0 + 1; a += blockDim.x) copy(a, b, c);
-        return;
-    }
-    const int t = (r - nr1 - nr2) * blockDim.x + threadIdx.x;
-    if (t >= 2 * n1 * n2) return;
-    const int rest = t >> 1;
-    copy((t & 1) ? n0 + 1 : 0, rest % n1 + 1, rest / n1 + 1);
+    const int T = 3 - D;
+    const unsigned nt = (unsigned)L.n(T), e = blockIdx.x * 256 + threadIdx.x;
+    const unsigned q = e / nt;
+    if (q >= 8u * Q) return;
+    const unsigned l = q / 8;
+    const int n = L.n(D), w = (int)(q & 3);
+    int x[3];
+    x[0] = (q & 4) ? L.nx + 1 : 0;
+    x[D] = w == 0 ? 0 : w == 1 ? 1 : w == 2 ? n : n + 1;
+    x[T] = (int)(e - q * nt) + 1;
+    const size_t o = (size_t)l * (size_t)L.plane + (size_t)L.cell(x[0], x[1], x[2]);
+    static_cast<raw*>(dst)[o] = static_cast<const raw*>(src)[o];
 }
 
 // ------------------------------------------------------------------------------------------

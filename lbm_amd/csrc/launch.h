@@ -158,15 +158,9 @@ struct Launch {
         }
     }
 
-    static hipError_t ghost_copy(const Layout& L, const void* src, void* dst, hipStream_t s) {
-        const int per[3] = {L.per_i, L.per_j, L.per_k};
-        const int n1 = L.n(L.ax1), n2 = L.n(L.ax2);
-        const int nr1 = per[L.ax1] ? 0 : 2 * (n2 + 2);
-        const int nr2 = per[L.ax2] ? 0 : 2 * n1;
-        const long long ne = per[L.ax0] ? 0 : 2LL * n1 * n2;
-        const long long blocks = nr1 + nr2 + (ne + 255) / 256;
-        if (blocks == 0) return hipSuccess;
-        hipLaunchKernelGGL((ghost_copy_kernel<Q, C>), dim3((unsigned)blocks), dim3(256), 0, s, L, src, dst, nr1, nr2);
+    static hipError_t ghost_keep(const Layout& L, const void* src, void* dst, int D, hipStream_t s) {
+        const unsigned blocks = (8u * Q * (unsigned)L.n(3 - D) + 255) / 256;
+        hipLaunchKernelGGL((ghost_keep_kernel<Q, C>), dim3(blocks), dim3(256), 0, s, L, src, dst, D);
         return hipGetLastError();
     }
 
@@ -442,7 +436,7 @@ struct Launch {
                               &averages_out, &field_in, &feq_init, &totals, &average,
                               sizeof(MemberTab<R>), &ens_pack, &ens_step,
                               kAdj ? &adj_step : nullptr, kAdj ? &adj_inflow : nullptr, kAdj ? &adj_face : nullptr,
-                              &objective, &halo_pack, &halo_unpack, &ghost_copy, &turb_step, (int)sizeof(R),
+                              &objective, &halo_pack, &halo_unpack, &ghost_keep, &turb_step, (int)sizeof(R),
                               (int)sizeof(typename C::raw)};
         return &o;
     }
