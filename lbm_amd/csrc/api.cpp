@@ -967,26 +967,22 @@ int lbm_generate_turbulence(lbm_ctx* c, int nrturb, double ampl, uint64_t seed, 
     if (c->d.iturb_pos < 1 || c->d.iturb_pos > c->d.nx) return fail(c, LBM_EINVAL, "iturb_pos outside the grid");
     const lbm_desc& d = c->d;
     const size_t n = (size_t)d.ny * d.nz * (nrturb + 1);
-    DevBuf scratch, out;
-    int rc = LBM_OK;
-    if ((rc = dev_alloc(c, scratch, turbulence_scratch_bytes(d.ny, d.nz, nrturb))) ||
-        (rc = dev_alloc(c, out, 4 * n * rb))) {
-        dev_free(scratch);
-        dev_free(out);
-        return rc;
-    }
+    // scratch and fields lie in the context's staging buffer (a window's fields are drawn every nrturb steps)
+    const size_t sb = turbulence_scratch_bytes(d.ny, d.nz, nrturb);
+    if (int rc = dev_alloc(c, c->stage, sb + 4 * n * rb)) return rc;
+    char* const out = static_cast<char*>(c->stage.p) + sb;
     auto run = [&]() -> int {
-        HIPCHK(c, turbulence_generate(rb, d.ny, d.nz, nrturb, seed, scratch.p, out.p, c->stream));
+        HIPCHK(c, turbulence_generate(rb, d.ny, d.nz, nrturb, seed, c->stage.p, out, c->stream));
         for (int q = 0; q < 3; ++q) {
             if (int r = dev_alloc(c, c->turb[q], n * rb)) return r;
-            HIPCHK(c, hipMemcpyAsync(c->turb[q].p, static_cast<char*>(out.p) + q * n * rb, n * rb,
+            HIPCHK(c, hipMemcpyAsync(c->turb[q].p, out + q * n * rb, n * rb,
                                      hipMemcpyDeviceToDevice, c->stream));
         }
         void* host[4] = {uu, vv, ww, rr};
         std::vector<unsigned char> img(n * rb);
         for (int q = 0; q < 4; ++q) {
             if (!host[q]) continue;
-            HIPCHK(c, hipMemcpyAsync(img.data(), static_cast<char*>(out.p) + q * n * rb, n * rb, hipMemcpyDeviceToHost,
+            HIPCHK(c, hipMemcpyAsync(img.data(), out + q * n * rb, n * rb, hipMemcpyDeviceToHost,
                                      c->stream));
             HIPCHK(c, hipStreamSynchronize(c->stream));
             for (size_t e = 0; e < n; ++e) {
@@ -998,10 +994,7 @@ int lbm_generate_turbulence(lbm_ctx* c, int nrturb, double ampl, uint64_t seed, 
         HIPCHK(c, hipStreamSynchronize(c->stream));
         return LBM_OK;
     };
-    rc = run();
-    dev_free(scratch);
-    dev_free(out);
-    if (rc) return rc;
+    if (int rc = run()) return rc;
     c->nrturb = nrturb;
     c->ampl = round_real(c, ampl);
     c->has_turb = true;
