@@ -5,7 +5,10 @@
 // Measured with 8 threads and 2 MiB slots, FP32 384x192x128: moments (154 MB) 15.6 -> 4.5 ms, a D3Q27
 // record (1.04 GB) out 97 -> 26.5 ms, in 35 -> 27 ms.  What fits one slot takes one copy on the calling
 // thread, also where it goes to several arrays (60x14x5 moments 123 -> 38 us), and spares the runtime's
-// page-locking of the caller's array on the way in (60x14x5 record 340 -> 70 us).
+// page-locking of the caller's array on the way in (60x14x5 record 340 -> 70 us).  The first copies through a
+// new pool cost up to 2.3 ms more, as its pages are touched (equilibrium start of 112x84x70 cells, 22 MB in: 3.4
+// ms, 1.1 ms from then on; the runtime's copies 1.6 and 1.1 ms).  Slots of 1 MiB halve that, but made a readout
+// of 154 MB 0.8 ms slower.
 #include "transfer.h"
 
 #include <hip/hip_runtime.h>
