@@ -296,7 +296,7 @@ StepHost step_host(const lbm_ctx* c, bool fold) {
 int step_buffers(lbm_ctx* c, const void* src, void* dst, int it) {
     StepHost h = step_host(c, c->fold_on);
     if (c->inflow_fold_on) {
-        h.inflow_fold = 1;
+        h.inflow_fold = c->inflow_fold_on;
         h.shear = c->shear.p;
         h.rho0 = c->d.rho0;
         inflow_values(c, it, &h.utime, &h.cosd, &h.sind);
@@ -310,7 +310,7 @@ int step_buffers(lbm_ctx* c, const void* src, void* dst, int it) {
 
 // boundarycond(f1, f2) for the non-periodic directions (src/m_boundarycond.F90:166-365).
 // skip_dir: a closed axis whose face pass the step kernel has already performed.
-int boundary(lbm_ctx* c, void* f1, const void* f2, int it, int skip_dir, bool skip_inflow, bool timed) {
+int boundary(lbm_ctx* c, void* f1, const void* f2, int it, int skip_dir, int inflow_fold, bool timed) {
     const lbm_desc& d = c->d;
     BoundaryHost h{};
     h.f1 = f1;
@@ -323,7 +323,7 @@ int boundary(lbm_ctx* c, void* f1, const void* f2, int it, int skip_dir, bool sk
         any = any || h.opt_lo[a] != 0;
     }
     h.inflow = d.ibnd == 1;
-    h.do_inflow = h.inflow && !skip_inflow;
+    h.do_inflow = !h.inflow ? 0 : inflow_fold == 0 ? 1 : inflow_fold == 2 ? 2 : 0;
     if (!any && !h.do_inflow) return LBM_OK;
     h.edges = edge_list(d);
     if (h.do_inflow) {
@@ -462,9 +462,13 @@ int lbm_create(const lbm_desc* desc, lbm_ctx** out) {
     {
         // With one closed axis (no edges, corners or snapshots then) the step kernel can perform
         // that axis's face pass itself, and with at most that one closed axis the inflow/outflow
-        // planes of i as well: a step is then one launch.  Ensembles always fold the face (a
-        // member's face must not need a launch of its own).  LBM_FOLD=0 selects the separate
-        // boundary kernels for a single domain.
+        // planes of i as well: a step is then one launch.  With two closed axes the inflow/outflow planes
+        // are the step kernel's but for the rows along the walls, from planes of 4096 cells on: measured on
+        // MI355X, FP32, separate -> in the step, us per step: D3Q27 250x98x70 90.1 -> 84.0, 60x150x120
+        // 89.8 -> 62.8, 300x150x90 197 -> 192, but 100x61x45 26.7 -> 25.9 (D3Q19 19.7 -> 20.6) and 30x16x14
+        // 8.8 -> 11.0, where the scattered stores at the end of a wave are the step's latency; FP16 alike,
+        // FP64 -1 to +12 %.  Ensembles always fold the face (a member's face must not need a launch of its
+        // own).  LBM_FOLD=0 selects the separate boundary kernel for a single domain.
         const int codes[3] = {d.ibnd, d.jbnd, d.kbnd};
         int nclosed = 0, cl = -1;
         for (int a = 0; a < 3; ++a)
@@ -474,10 +478,15 @@ int lbm_create(const lbm_desc* desc, lbm_ctx** out) {
         // halo domains always fold: the separate boundary kernels do not know halo planes
         const bool fold = d.jbnd == LBM_BND_HALO || (fv ? atoi(fv) != 0 : kFoldDefault);
         c->fold_on = c->fold_dir >= 0 && fold;
-        c->inflow_fold_on = d.ibnd == 1 && fold && (nclosed == 0 || c->fold_on);
+        const bool wide = (long long)d.ny * d.nz >= 4096;
+        c->inflow_fold_on = d.ibnd != 1 || !fold ? 0 : nclosed < 2 ? 1 : wide ? 2 : 0;
         // LBM_INFLOW_FOLD=0 keeps the face folded but writes the inflow/outflow planes with their own
         // kernel (measured slower: tile 384x24x128 14.0 k vs 16.2 k MLUPS, whole domain -1 %)
-        if (const char* iv = getenv("LBM_INFLOW_FOLD")) c->inflow_fold_on = c->inflow_fold_on && atoi(iv) != 0;
+        // LBM_INFLOW_FOLD=1 folds them with two closed axes whatever the size
+        if (const char* iv = getenv("LBM_INFLOW_FOLD")) {
+            if (atoi(iv) == 0) c->inflow_fold_on = 0;
+            else if (d.ibnd == 1 && fold && nclosed == 2) c->inflow_fold_on = 2;
+        }
     }
     hipGetDevice(&c->device);
     // lbm_get_totals_noalloc's scratch on this device (a failed lookup is reported by that call)
@@ -610,7 +619,7 @@ namespace {
 StepHost step_base(lbm_ctx* c) {
     StepHost h = step_host(c, c->fold_on);
     if (c->inflow_fold_on) {
-        h.inflow_fold = 1;
+        h.inflow_fold = c->inflow_fold_on;
         h.shear = c->shear.p;
         h.rho0 = c->d.rho0;
         h.heavy_first |= c->lay.ax1 == 0 ? 1 : c->lay.ax2 == 0 ? 2 : 0;

@@ -71,8 +71,9 @@ struct lbm_ctx {
     int fold_dir = -1;             // the only closed axis (-1: none or several): its face pass can
                                    // run inside the step kernel (always in ensembles)
     bool fold_on = false;          // single-domain steps fold it
-    bool inflow_fold_on = false;   // single-domain steps write the inflow/outflow planes of i in the
-                                   // step kernel (with fold_on, or with no closed axis)
+    int inflow_fold_on = 0;        // single-domain steps write the inflow/outflow planes of i in the step
+                                   // kernel: 1 with fold_on or no closed axis, 2 with two closed axes and wide planes
+                                   // (not the rows along their walls)
     int variant = 1;               // step-kernel variant (LBM_STEP_VARIANT), see impl.h; non-temporal
     int step_lds = 0;              // dynamic LDS bytes per step-kernel block (residency cap), see lbm_create
                                    // stores measured fastest on MI355X (5.32 vs 5.11 TB/s)
@@ -120,8 +121,8 @@ void inflow_values(const lbm_ctx* c, int it, double* ut, double* cs, double* sn)
 // performs the face pass of c->fold_dir
 lbm::StepHost step_host(const lbm_ctx* c, bool fold);
 // boundarycond(f1, f2) for the non-periodic directions; skip_dir: face done by the step kernel;
-// skip_inflow: inflow/outflow planes done by the step kernel
-int boundary(lbm_ctx* c, void* f1, const void* f2, int it, int skip_dir = -1, bool skip_inflow = false,
+// inflow_fold: what of the inflow/outflow planes the step kernel did (StepArgs::inflow_fold)
+int boundary(lbm_ctx* c, void* f1, const void* f2, int it, int skip_dir = -1, int inflow_fold = 0,
              bool timed = false);
 // one step (iteration it) from buffer src into buffer dst, which holds the ghosts of the state
 // before src; the context's own buffers are not touched

@@ -20,12 +20,26 @@ struct EdgeList {
     int mir[20][3];
 };
 
+// Rows of the inflow planes along the walls of two closed axes, of n0, n1 >= 2 cells: the two walls of the
+// second, then those of the first between them.  Cell e (0-based) of them -> its coordinates.
+__host__ __device__ inline int inflow_rim_cells(int n0, int n1) { return 2 * n0 + 2 * (n1 - 2); }
+__host__ __device__ inline void inflow_rim_cell(int e, int n0, int n1, int& x0, int& x1) {
+    if (e < 2 * n0) {
+        x0 = (e < n0 ? e : e - n0) + 1;
+        x1 = e < n0 ? 1 : n1;
+    } else {
+        x0 = (e & 1) ? n0 : 1;
+        x1 = ((e - 2 * n0) >> 1) + 2;
+    }
+}
+
 // The boundary passes of one step that the step kernel does not perform.
 struct BoundaryHost {
     void* f1;
     const void* f2;
     int opt_lo[3], opt_hi[3];   // wall options of the closed axes (0: not closed, or not this launch's)
-    int inflow, do_inflow;      // i has inflow/outflow planes; they are this launch's
+    int inflow, do_inflow;      // i has inflow/outflow planes; they are this launch's (2: their rows
+                                // along the walls of j and k are)
     const void* shear;          // uvel_shear(nz) (compute type)
     double utime, cosd, sind, rho0;
     EdgeList edges;
@@ -52,7 +66,7 @@ struct StepHost {
     void* avg;            // averaging sums (6 cell planes of the compute type) or nullptr
     void* tau_out;
     int fold_dir, fold_opt_lo, fold_opt_hi;   // closed face performed by the step kernel
-    int inflow_fold;                          // inflow/outflow planes performed by the step kernel
+    int inflow_fold;                          // inflow/outflow planes performed by the step kernel (StepArgs)
     const void* shear;                        // uvel_shear(nz) (compute type)
     double utime, cosd, sind, rho0;           // inflow values of the step
     int heavy_first;                          // bit 0 / 1: cells 1 and n of ax1 / ax2 first

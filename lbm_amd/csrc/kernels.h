@@ -59,7 +59,8 @@ struct StepArgs {
     R* tau_out;            // cell layout; nullptr: tau not stored
     int fold_dir;          // closed axis whose face pass this kernel performs (-1: none)
     int fold_opt_lo, fold_opt_hi;
-    // inflow/outflow planes of i written by the cells at i = 1 and i = nx (0: separate pass)
+    // inflow/outflow planes of i written by the cells at i = 1 and i = nx (0: separate pass; 2: but for
+    // the rows along the walls of j and k, both closed, whose ghosts the face passes read first)
     int inflow_fold;
     const R* shear;        // uvel_shear(nz)
     R utime, cosd, sind, rho0;
@@ -595,7 +596,8 @@ __device__ __forceinline__ void fold_boundaries(const StepArgs<typename C::real>
     using Lt = Lattice<Q>;
     const Layout& L = a.lay;
     raw* __restrict__ f1 = static_cast<raw*>(a.dst);
-    const bool at_end = a.inflow_fold && (i == 1 || i == L.nx);
+    const bool at_end = a.inflow_fold && (i == 1 || i == L.nx) &&
+                        (a.inflow_fold == 1 || (j > 1 && j < L.ny && k > 1 && k < L.nz));
     if (a.fold_dir == 0) {
         if (i == 1) fold_face<Q, C, 0, 0>(a, i, j, k, oc, false, dev);
         if (i == L.nx) fold_face<Q, C, 0, 1>(a, i, j, k, oc, false, dev);
@@ -865,6 +867,7 @@ struct BoundaryArgs {
     int ta[3];                 // the face's axis that is stored first
     int inflow;                // i has inflow/outflow planes
     int inflow_blocks;         // their blocks; 0: not this launch's
+    int inflow_rim;            // only their rows along the walls of j and k
     const R* shear;            // uvel_shear(nz)
     R utime, cosd, sind, rho0;
     EdgeList edges;
@@ -898,7 +901,10 @@ __device__ __forceinline__ void st(const Layout& L, void* f, int l, int off, typ
 //     call, which the thread that replaces it passes on first;
 //   * S on an inflow plane and a closed axis at once: no pass writes it.
 // Measured on MI355X, FP32, per step: closed box 101x61x45 (three closed axes) 38.4 us in four launches
-// -> 7.9 us; duct 250x98x70 (inflow, two closed axes) 52.1 us in four launches -> 25.5 us.
+// -> 7.9 us; duct 250x98x70 (inflow, two closed axes) 52.1 us in four launches -> 25.5 us.  The inflow planes
+// were most of the duct's: with i contiguous, four lines for every value.  Now the step kernel's end cells
+// write them but for the rows along the walls (inflow_fold = 2), and the launch takes 11.6 us; the
+// two kernels of a step 92 -> 89.5 us.
 template <int Q, class C>
 __global__ void __launch_bounds__(256) boundary_kernel(const BoundaryArgs<typename C::real> a) {
     using R = typename C::real;
@@ -991,14 +997,18 @@ __global__ void __launch_bounds__(256) boundary_kernel(const BoundaryArgs<typena
     // ---- inflow/outflow planes: (along the plane, population)
     if (b < a.inflow_blocks) {
         const int T0 = a.ta[0], T1 = 3 - T0;
-        const int area = n[T0] * n[T1];
+        const int area = a.inflow_rim ? inflow_rim_cells(n[T0], n[T1]) : n[T0] * n[T1];
         const int per_pop = (area + 255) / 256;
         const int l = b / per_pop;
         const int e = (b - l * per_pop) * 256 + threadIdx.x;
         if (e >= area) return;
         int x[3];
-        x[T1] = e / n[T0] + 1;
-        x[T0] = e - (x[T1] - 1) * n[T0] + 1;
+        if (a.inflow_rim) {
+            inflow_rim_cell(e, n[T0], n[T1], x[T0], x[T1]);
+        } else {
+            x[T1] = e / n[T0] + 1;
+            x[T0] = e - (x[T1] - 1) * n[T0] + 1;
+        }
         const int cx = Lattice<Q>::cx(l);
         const int src = cx <= 0 ? l : Lattice<Q>::opposite(l);
         x[0] = 1;

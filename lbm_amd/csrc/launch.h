@@ -236,7 +236,8 @@ struct Launch {
             a.face_blocks[d] = a.face[d] ? (int)(area * 2 * Outgoing<Q>::count) : 0;
             blocks += a.face_blocks[d];
             if (d == 0 && h.do_inflow) {
-                a.inflow_blocks = (int)(area * Q);
+                a.inflow_rim = h.do_inflow == 2;
+                a.inflow_blocks = (int)((a.inflow_rim ? (inflow_rim_cells(L.n(a.ta[0]), L.n(t1)) + 255) / 256 : area) * Q);
                 blocks += a.inflow_blocks;
             }
         }
