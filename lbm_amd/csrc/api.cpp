@@ -549,7 +549,7 @@ int lbm_destroy(lbm_ctx* c) {
     DevBuf* all[] = {&c->ablvisc, &c->shear, &c->solid, &c->turb[0], &c->turb[1], &c->turb[2], &c->force[0],
                      &c->force[1], &c->force[2], &c->tau, &c->ext[0], &c->ext[1], &c->ext[2], &c->ext[3],
                      &c->stage, &c->partial, &c->t_rot, &c->t_theta, &c->t_blade, &c->t_nfoil,
-                     &c->t_nang, &c->t_foil, &c->t_pts, &c->theta, &c->adj_ck, &c->adj_snaps,
+                     &c->t_nang, &c->t_foil, &c->t_pts, &c->theta, &c->avg, &c->adj_ck, &c->adj_snaps,
                      &c->adj_lam, &c->adj_gF, &c->adj_gS, &c->adj_acc};
     for (DevBuf* b : all) dev_free(*b);
     for (hipEvent_t ev : c->ev_step) hipEventDestroy(ev);
