@@ -121,7 +121,9 @@ int lbm_set_turbulence(lbm_ctx* ctx, const void* uu, const void* vv, const void*
  * deviation.  The random phases come from SplitMix64(seed) where the reference calls the
  * compiler's random_number.  The fields become the context's turbulence forcing (as
  * lbm_set_turbulence with ampl); uu, vv, ww, rr (ny,nz,0:nrturb) receive copies when not NULL
- * (the turbulence restart record).  FP32/FP64 compute only. */
+ * (the turbulence restart record).  FP32/FP64 compute only.  The call's device scratch (per slice and
+ * variable about ny*nz complex FP64 values and the fields) stays with the context where it is no larger
+ * than a record of the state, and is freed when the call returns otherwise. */
 int lbm_generate_turbulence(lbm_ctx* ctx, int nrturb, double ampl, uint64_t seed, void* uu, void* vv,
                             void* ww, void* rr, int realkind);
 /* external_forcing(3,0:nx+1,0:ny+1,0:nz+1) applied every step by forcings_apply

@@ -976,9 +976,12 @@ int lbm_generate_turbulence(lbm_ctx* c, int nrturb, double ampl, uint64_t seed, 
     if (c->d.iturb_pos < 1 || c->d.iturb_pos > c->d.nx) return fail(c, LBM_EINVAL, "iturb_pos outside the grid");
     const lbm_desc& d = c->d;
     const size_t n = (size_t)d.ny * d.nz * (nrturb + 1);
-    // scratch and fields lie in the context's staging buffer (a window's fields are drawn every nrturb steps)
-    const size_t sb = turbulence_scratch_bytes(d.ny, d.nz, nrturb);
-    if (int rc = dev_alloc(c, c->stage, sb + 4 * n * rb)) return rc;
+    // Scratch and fields lie in the context's staging buffer (a window's fields are drawn every nrturb steps).  It
+    // stays with the context up to the size that a record of the state takes there; what a longer window needs
+    // beyond that (2 GB for 1000 slices of 192x128) goes when the call returns.
+    const size_t sb = turbulence_scratch_bytes(d.ny, d.nz, nrturb), need = sb + 4 * n * rb;
+    const bool give_back = need > c->stage.n && need > ncell_padded(c) * d.q * rb;
+    if (int rc = dev_alloc(c, c->stage, need)) return rc;
     char* const out = static_cast<char*>(c->stage.p) + sb;
     auto run = [&]() -> int {
         HIPCHK(c, turbulence_generate(rb, d.ny, d.nz, nrturb, seed, c->stage.p, out, c->stream));
@@ -1003,7 +1006,12 @@ int lbm_generate_turbulence(lbm_ctx* c, int nrturb, double ampl, uint64_t seed, 
         HIPCHK(c, hipStreamSynchronize(c->stream));
         return LBM_OK;
     };
-    if (int rc = run()) return rc;
+    const int rc = run();
+    if (give_back) {
+        (void)hipStreamSynchronize(c->stream);
+        dev_free(c->stage);
+    }
+    if (rc) return rc;
     c->nrturb = nrturb;
     c->ampl = round_real(c, ampl);
     c->has_turb = true;

@@ -30,3 +30,18 @@ def test_averaging_sums_are_freed():
         held.append(free_bytes())
     # from the second context on nothing is set up any more; each lost sums would take 40 MB
     assert sums > SLACK and held[0] - held[-1] < SLACK
+
+
+def test_window_scratch_is_given_back():
+    """A window whose scratch and fields outgrow a record of the state: what stays is what the context needs
+    afterwards (populations, the three fields, at most a record's staging memory)."""
+    dims, n, window = (16, 128, 128), 200, 201 * 128 * 128 * 4
+    record = 19 * np.prod([x + 2 for x in dims]) * 4
+    before = free_bytes()
+    with Domain(19, dims, "f32", ibgk=2, kinevisc=0.1, ibnd=1, kbnd=12) as d:
+        for seed in (1, 2):
+            d.generate_turbulence(n, 1e-3, seed, return_fields=False)
+            held = before - free_bytes()
+            print(f"seed {seed}: {held >> 20} MB held", flush=True)
+            # scratch (4 variables of 201 x 65 x 256 complex values) and fields took 267 MB more
+            assert held < d.info()["device_bytes"] + 3 * window + record + SLACK
