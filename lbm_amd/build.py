@@ -18,6 +18,7 @@ CSRC = os.path.join(HERE, "csrc")
 BUILD = os.path.join(HERE, "_build")
 LIB = os.path.join(HERE, "liblbm_hip.so")
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
+CXX = os.environ.get("CXX", "g++")
 FLANG = os.environ.get("FLANG", "/opt/rocm/bin/amdflang")
 FORTRAN = os.path.join(HERE, "fortran")
 ARCH = "gfx950"
@@ -62,6 +63,11 @@ def build(verbose: bool = False) -> str:
     subprocess.run([HIPCC] + FLAGS + ["-x", "hip", "-o", os.path.join(BUILD, "layout_check"),
                                       os.path.join(CSRC, "layout_check.cpp")],
                    check=True, stdout=subprocess.DEVNULL, stderr=subprocess.DEVNULL)
+    # host-only check of the copies to and from the caller's arrays, with a stand-in for the runtime
+    subprocess.run([CXX, "-O2", "-std=c++17", "-Wall", "-pthread", "-D__HIP_PLATFORM_AMD__", "-I", CSRC,
+                    "-I", os.path.join(os.path.dirname(os.path.dirname(HIPCC)), "include"),
+                    "-o", os.path.join(BUILD, "transfer_check"), os.path.join(CSRC, "transfer_check.cpp"),
+                    os.path.join(CSRC, "transfer.cpp")], check=True)
     tmp = LIB + ".tmp"
     cmd = [HIPCC, "-shared", "-fPIC", f"--offload-arch={ARCH}", "-o", tmp] + objs
     subprocess.run(cmd, check=True)

@@ -18,8 +18,8 @@
 #include <condition_variable>
 #include <cstring>
 #include <exception>
-#include <memory>
 #include <mutex>
+#include <new>
 #include <thread>
 
 namespace lbm_host {
@@ -41,14 +41,31 @@ struct Job {
     int np;
     bool in;             // host to device
     size_t total, chunks;
+    int threads;
     std::atomic<size_t> next{0};
     std::atomic<int> error{hipSuccess};
-    // threads that take part; none joins any more once the calling thread has run out of chunks
-    std::mutex mu;
-    std::condition_variable idle;
-    int active = 0;
-    bool closed = false;
 };
+
+// The threads that take part in large copies beside the calling one.  They stay until the last context goes and
+// are joined then: nothing of a thread outlives its contexts.  A copy does not wait for a thread that wakes late
+// (other threads of the process may keep all processors busy): it finds the job gone.  Threads started and
+// joined by each copy made copies of 16 MB slower than the runtime's beside a spinning OpenMP team.  Never
+// destroyed: a program may exit with contexts alive, whose threads then still wait here.
+struct Team {
+    std::thread th[kWorkers - 1];
+    int started = 0;             // guarded by g_mu
+    std::mutex mu;
+    std::condition_variable wake, idle;
+    Job* job = nullptr;
+    unsigned long long turn = 0;
+    int active = 0;
+    bool stop = false;
+};
+Team& team() {
+    alignas(Team) static unsigned char place[sizeof(Team)];
+    static Team* const t = new (place) Team;
+    return *t;
+}
 
 // Everything of the device range's chunk k that a part holds or wants, from or to the slot.
 void move_host(const Job& j, size_t k, char* slot) {
@@ -109,23 +126,57 @@ void work(Job& j, int w) {
         if (e) (void)hipEventDestroy(e);
 }
 
-// A thread of the team.  One that the system starts late (other threads of the process may keep all
-// processors busy) finds the job closed, and nobody waits for it: joined threads made copies of 16 MB
-// slower than the runtime's beside a spinning OpenMP team.
-void join_in(std::shared_ptr<Job> j, int w) {
-    {
-        std::lock_guard<std::mutex> lk(j->mu);
-        if (j->closed) return;
-        ++j->active;
+void member(Team* t, int w) {
+    unsigned long long seen = 0;
+    std::unique_lock<std::mutex> lk(t->mu);
+    for (;;) {
+        t->wake.wait(lk, [&] { return t->stop || (t->job && t->turn != seen); });
+        if (t->stop) return;
+        seen = t->turn;
+        Job& j = *t->job;
+        if (w >= j.threads) continue;
+        ++t->active;
+        lk.unlock();
+        work(j, w);
+        lk.lock();
+        if (--t->active == 0) t->idle.notify_all();
     }
-    work(*j, w);
-    std::lock_guard<std::mutex> lk(j->mu);
-    if (--j->active == 0) j->idle.notify_all();
+}
+
+// The job by up to j.threads threads, this one among them.  g_mu is held.
+void work_together(Job& j) {
+    Team& t = team();
+    try {
+        for (; t.started < j.threads - 1; ++t.started) t.th[t.started] = std::thread(member, &t, t.started + 1);
+    } catch (const std::exception&) {
+        // fewer threads than wanted: the others take their chunks
+    }
+    {
+        std::lock_guard<std::mutex> lk(t.mu);
+        t.job = &j;
+        ++t.turn;
+    }
+    t.wake.notify_all();
+    work(j, 0);
+    std::unique_lock<std::mutex> lk(t.mu);
+    t.job = nullptr;   // nobody joins any more
+    t.idle.wait(lk, [&] { return t.active == 0; });
+}
+
+// g_mu is held: no copy is under way.
+void dismiss() {
+    Team& t = team();
+    {
+        std::lock_guard<std::mutex> lk(t.mu);
+        t.stop = true;
+    }
+    t.wake.notify_all();
+    for (; t.started > 0; --t.started) t.th[t.started - 1].join();
+    t.stop = false;
 }
 
 int copy(lbm_ctx* c, char* dev, const HostPart* parts, int n, bool in) {
-    const std::shared_ptr<Job> job = std::make_shared<Job>();
-    Job& j = *job;
+    Job j;
     j.c = c;
     j.dev = dev;
     j.parts = parts;
@@ -160,18 +211,8 @@ int copy(lbm_ctx* c, char* dev, const HostPart* parts, int n, bool in) {
         return LBM_OK;
     }
     // a thread costs about as much as emptying a slot: one for every two chunks
-    const int threads = (int)std::min<size_t>(kWorkers, (j.chunks + 1) / 2);
-    try {
-        for (int w = 1; w < threads; ++w) std::thread(join_in, job, w).detach();
-    } catch (const std::exception&) {
-        // fewer threads than wanted: the others take their chunks
-    }
-    work(j, 0);
-    {
-        std::unique_lock<std::mutex> lk(j.mu);
-        j.closed = true;
-        j.idle.wait(lk, [&] { return j.active == 0; });
-    }
+    j.threads = (int)std::min<size_t>(kWorkers, (j.chunks + 1) / 2);
+    work_together(j);
     if (j.error.load() != hipSuccess) {
         (void)hipStreamSynchronize(c->stream);   // nothing still uses the slots
         return hipfail(c, (hipError_t)j.error.load(), in ? "copy to the device" : "copy to the host");
@@ -190,6 +231,7 @@ void transfer_release() {
     std::lock_guard<std::mutex> lk(g_users_mu);
     if (--g_users > 0) return;
     std::lock_guard<std::mutex> lk2(g_mu);
+    dismiss();
     if (g_slots) (void)hipHostFree(g_slots);
     g_slots = nullptr;
 }

@@ -1,0 +1,215 @@
+// CPU check of the copies to and from the caller's arrays (transfer.cpp), linked against the stand-in for the
+// HIP runtime below: copies are memory copies on the calling thread, page-locked memory is ordinary memory that
+// is counted, events and streams are names.
+//
+//   transfer_check <case>    prints one JSON line, exits 0 if the case holds
+#include <hip/hip_runtime.h>
+
+#include <algorithm>
+#include <atomic>
+#include <chrono>
+#include <cstdio>
+#include <cstdlib>
+#include <cstring>
+#include <functional>
+#include <map>
+#include <mutex>
+#include <random>
+#include <string>
+#include <thread>
+#include <vector>
+
+#include "transfer.h"
+
+using namespace lbm_host;
+
+namespace {
+
+// ---- the stand-in runtime
+thread_local int t_device = 0;
+std::atomic<int> g_threads_seen{0}, g_threads_ended{0};
+struct ThreadState {   // what a runtime keeps per thread, released some time after the thread's function
+    bool used = false;
+    ~ThreadState() {
+        if (!used) return;
+        std::this_thread::sleep_for(std::chrono::milliseconds(100));
+        ++g_threads_ended;
+    }
+};
+thread_local ThreadState t_state;
+
+std::mutex g_lock_mu;
+std::map<void*, size_t> g_locked;
+size_t g_locked_bytes = 0;
+std::atomic<bool> g_no_lock{false};
+std::atomic<int> g_fail_after{-1};   // copies until one fails; -1: none does
+std::function<void(const void*, const void*, size_t)> g_on_copy;
+
+}  // namespace
+
+extern "C" {
+hipError_t hipSetDevice(int d) {
+    if (!t_state.used) {
+        t_state.used = true;
+        ++g_threads_seen;
+    }
+    t_device = d;
+    return hipSuccess;
+}
+hipError_t hipGetDevice(int* d) {
+    *d = t_device;
+    return hipSuccess;
+}
+hipError_t hipEventCreateWithFlags(hipEvent_t* e, unsigned) {
+    *e = reinterpret_cast<hipEvent_t>(std::malloc(1));
+    return hipSuccess;
+}
+hipError_t hipEventDestroy(hipEvent_t e) {
+    std::free(e);
+    return hipSuccess;
+}
+hipError_t hipEventRecord(hipEvent_t, hipStream_t) { return hipSuccess; }
+hipError_t hipEventSynchronize(hipEvent_t) { return hipSuccess; }
+hipError_t hipStreamSynchronize(hipStream_t) { return hipSuccess; }
+hipError_t hipGetLastError() { return hipSuccess; }
+const char* hipGetErrorString(hipError_t) { return "an error"; }
+hipError_t hipMemcpyAsync(void* dst, const void* src, size_t n, hipMemcpyKind, hipStream_t) {
+    if (g_on_copy) g_on_copy(dst, src, n);
+    if (g_fail_after.load() >= 0 && g_fail_after.fetch_sub(1) == 0) return hipErrorUnknown;
+    std::memcpy(dst, src, n);
+    return hipSuccess;
+}
+hipError_t hipHostMalloc(void** p, size_t n, unsigned) {
+    if (g_no_lock.load()) return hipErrorOutOfMemory;
+    std::lock_guard<std::mutex> lk(g_lock_mu);
+    *p = std::malloc(n);
+    g_locked[*p] = n;
+    g_locked_bytes += n;
+    return hipSuccess;
+}
+hipError_t hipHostFree(void* p) {
+    std::lock_guard<std::mutex> lk(g_lock_mu);
+    g_locked_bytes -= g_locked[p];
+    g_locked.erase(p);
+    std::free(p);
+    return hipSuccess;
+}
+}
+
+namespace lbm_host {
+int hipfail(lbm_ctx*, hipError_t, const char*) { return LBM_EHIP; }
+}  // namespace lbm_host
+
+namespace {
+
+constexpr size_t kMB = 1u << 20;
+
+std::vector<unsigned char> noise(size_t n, unsigned seed) {
+    std::vector<unsigned char> v(n);
+    std::mt19937_64 g(seed);
+    for (size_t q = 0; q < n; q += 8) {
+        const unsigned long long r = g();
+        std::memcpy(&v[q], &r, std::min<size_t>(8, n - q));
+    }
+    return v;
+}
+
+// A range of `sizes` one after the other; part q is the caller's unless wanted says otherwise.  Out of the device
+// and back in, with guards around every array.
+bool round_trip(lbm_ctx* c, const std::vector<size_t>& sizes, unsigned seed, unsigned unwanted) {
+    size_t total = 0;
+    std::vector<HostPart> parts;
+    std::vector<std::vector<unsigned char>> host;
+    for (size_t s : sizes) {
+        host.emplace_back(s + 128, (unsigned char)0xA5);
+        parts.push_back({nullptr, total, s});
+        total += s;
+    }
+    for (size_t q = 0; q < parts.size(); ++q)
+        if (!(unwanted >> q & 1)) parts[q].host = host[q].data() + 64;
+    std::vector<unsigned char> dev = noise(total, seed);
+    const std::vector<unsigned char> before = dev;
+    if (copy_out(c, dev.data(), parts.data(), (int)parts.size()) != LBM_OK || dev != before) return false;
+    for (size_t q = 0; q < parts.size(); ++q) {
+        const unsigned char* h = host[q].data();
+        for (int g = 0; g < 64; ++g)
+            if (h[g] != 0xA5 || h[64 + sizes[q] + g] != 0xA5) return false;
+        if (parts[q].host) {
+            if (std::memcmp(h + 64, before.data() + parts[q].offset, sizes[q]) != 0) return false;
+        } else if (std::count(h + 64, h + 64 + sizes[q], 0xA5) != (long)sizes[q]) {
+            return false;
+        }
+    }
+    if (unwanted) return true;   // what goes in covers the range
+    std::vector<unsigned char> to(total + 128, (unsigned char)0x5A);
+    if (copy_in(c, to.data() + 64, parts.data(), (int)parts.size()) != LBM_OK) return false;
+    for (int g = 0; g < 64; ++g)
+        if (to[g] != 0x5A || to[64 + total + g] != 0x5A) return false;
+    return std::memcmp(to.data() + 64, before.data(), total) == 0;
+}
+
+bool contents(lbm_ctx* c) {
+    const std::vector<std::vector<size_t>> sets = {
+        {1}, {100, 3, 7}, {2 * kMB}, {2 * kMB + 1}, {5 * kMB, 5 * kMB, 5 * kMB, 5 * kMB, 4},
+        {kMB - 4, 3 * kMB + 4, 1}, {70 * kMB + 12345}, {0, 10}};
+    for (size_t n = 0; n < sets.size(); ++n)
+        for (unsigned unwanted : {0u, 1u, 2u, 5u})
+            if (!round_trip(c, sets[n], (unsigned)n, unwanted)) return false;
+    return true;
+}
+
+// every copy that fails is reported, and the next one is whole
+bool errors(lbm_ctx* c) {
+    std::vector<unsigned char> host(20 * kMB), dev = noise(host.size(), 3);
+    for (size_t n : {kMB, 20 * kMB})
+        for (int after : {0, 1, 3, 9}) {
+            const HostPart part{host.data(), 0, n};
+            if ((size_t)after * 2 * kMB >= n) continue;
+            for (bool in : {false, true}) {
+                g_fail_after = after;
+                const int rc = in ? copy_in(c, dev.data(), &part, 1) : copy_out(c, dev.data(), &part, 1);
+                g_fail_after = -1;
+                if (rc != LBM_EHIP) return false;
+            }
+            if (!round_trip(c, {n}, 4, 0)) return false;
+        }
+    return true;
+}
+
+}  // namespace
+
+int main(int argc, char** argv) {
+    const std::string name = argc > 1 ? argv[1] : "";
+    lbm_ctx c;
+    bool ok = false;
+    if (name == "contents") {
+        transfer_retain();
+        ok = contents(&c);
+        transfer_release();
+        ok = ok && g_locked_bytes == 0;
+    } else if (name == "no_page_locked_memory") {
+        g_no_lock = true;
+        transfer_retain();
+        ok = contents(&c);
+        g_no_lock = false;
+        ok = ok && contents(&c);
+        transfer_release();
+    } else if (name == "errors") {
+        transfer_retain();
+        ok = errors(&c);
+        transfer_release();
+    } else if (name == "threads_end") {
+        // no thread that took part in a copy lives on after the last context, nor does its share of the runtime
+        for (int n = 0; n < 3; ++n) {
+            transfer_retain();
+            ok = round_trip(&c, {32 * kMB}, 5, 0);
+            transfer_release();
+            if (t_state.used) g_threads_seen = g_threads_seen.load() - 1, t_state.used = false;   // the caller's own
+            ok = ok && g_threads_ended == g_threads_seen;
+            if (!ok) break;
+        }
+    }
+    std::printf("{\"case\": \"%s\", \"ok\": %s, \"threads\": %d, \"ended\": %d, \"locked\": %zu}\n", name.c_str(),
+                ok ? "true" : "false", g_threads_seen.load(), g_threads_ended.load(), g_locked_bytes);
+    return ok ? 0 : 1;
+}
