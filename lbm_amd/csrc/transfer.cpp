@@ -95,7 +95,6 @@ void work(Job& j, int w) {
         return true;
     };
     hipEvent_t ev[2] = {nullptr, nullptr};
-    if (bad(hipSetDevice(j.c->device))) return;
     for (hipEvent_t& e : ev)
         if (bad(hipEventCreateWithFlags(&e, hipEventDisableTiming))) break;
     size_t held[2] = {0, 0};
@@ -137,7 +136,8 @@ void member(Team* t, int w) {
         if (w >= j.threads) continue;
         ++t->active;
         lk.unlock();
-        work(j, w);
+        // (a thread that cannot take the device leaves its chunks to the others)
+        if (hipSetDevice(j.c->device) == hipSuccess) work(j, w);
         lk.lock();
         if (--t->active == 0) t->idle.notify_all();
     }
@@ -175,6 +175,19 @@ void dismiss() {
     t.stop = false;
 }
 
+// The context's device is the calling thread's current one while this lives, and the caller's own again afterwards.
+struct OnDevice {
+    int mine = -1, own = -1;
+    hipError_t error;
+    explicit OnDevice(int d) : mine(d) {
+        error = hipGetDevice(&own);
+        if (error == hipSuccess && own != mine) error = hipSetDevice(mine);
+    }
+    ~OnDevice() {
+        if (own >= 0 && own != mine) (void)hipSetDevice(own);
+    }
+};
+
 int copy(lbm_ctx* c, char* dev, const HostPart* parts, int n, bool in) {
     Job j;
     j.c = c;
@@ -185,6 +198,8 @@ int copy(lbm_ctx* c, char* dev, const HostPart* parts, int n, bool in) {
     j.total = 0;
     for (int q = 0; q < n; ++q)
         if (parts[q].host) j.total = std::max(j.total, parts[q].offset + parts[q].bytes);
+    const OnDevice on(c->device);
+    HIPCHK(c, on.error);
     // what is queued ends before the slots are taken: others' copies do not wait for this context's steps
     HIPCHK(c, hipStreamSynchronize(c->stream));
     if (j.total == 0) return LBM_OK;

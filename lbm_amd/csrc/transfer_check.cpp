@@ -198,6 +198,20 @@ int main(int argc, char** argv) {
         transfer_retain();
         ok = errors(&c);
         transfer_release();
+    } else if (name == "device_of_the_caller") {
+        // a context on another device than the calling thread's current one: the copies are made with its device
+        // current, and the caller finds its own again
+        c.device = 1;
+        std::atomic<int> wrong{0};
+        g_on_copy = [&](const void*, const void*, size_t) { wrong += t_device != 1; };
+        transfer_retain();
+        ok = true;
+        for (size_t n : {kMB, 20 * kMB}) {
+            t_device = 0;
+            ok = ok && round_trip(&c, {n}, 6, 0) && t_device == 0;
+        }
+        transfer_release();
+        ok = ok && wrong == 0 && t_device == 0;
     } else if (name == "threads_end") {
         // no thread that took part in a copy lives on after the last context, nor does its share of the runtime
         for (int n = 0; n < 3; ++n) {
