@@ -448,7 +448,6 @@ int lbm_create(const lbm_desc* desc, lbm_ctx** out) {
     if (e != hipSuccess || ndev == 0) return fail(nullptr, LBM_EHIP, std::string("no HIP device: ") + hipGetErrorString(e));
 
     lbm_ctx* c = new lbm_ctx();
-    transfer_retain();
     c->d = d;
     c->d.block_x = bx;
     c->d.block_y = by;
@@ -489,6 +488,7 @@ int lbm_create(const lbm_desc* desc, lbm_ctx** out) {
         }
     }
     hipGetDevice(&c->device);
+    transfer_retain(c->device);
     // lbm_get_totals_noalloc's scratch on this device (a failed lookup is reported by that call)
     scratch_resolve(c->device);
     // Resident step-kernel blocks per CU, capped by reserving 1/n of the CU's LDS per block (the
@@ -555,7 +555,7 @@ int lbm_destroy(lbm_ctx* c) {
     for (hipEvent_t ev : c->ev_step) hipEventDestroy(ev);
     for (hipEvent_t ev : c->ev_bc) hipEventDestroy(ev);
     if (c->stream) hipStreamDestroy(c->stream);
-    transfer_release();
+    transfer_release(c->device);
     delete c;
     return LBM_OK;
 }

@@ -29,11 +29,6 @@ namespace {
 constexpr size_t kSlot = 2u << 20;   // bytes of a slot
 constexpr int kWorkers = 8;          // threads of a large copy, two slots each
 
-std::mutex g_mu;                     // one copy at a time: the link is one
-std::mutex g_users_mu;
-int g_users = 0;
-char* g_slots = nullptr;             // 2 * kWorkers slots (guarded by g_mu)
-
 struct Job {
     lbm_ctx* c;
     char* dev;
@@ -46,14 +41,13 @@ struct Job {
     std::atomic<int> error{hipSuccess};
 };
 
-// The threads that take part in large copies beside the calling one.  They stay until the last context goes and
-// are joined then: nothing of a thread outlives its contexts.  A copy does not wait for a thread that wakes late
-// (other threads of the process may keep all processors busy): it finds the job gone.  Threads started and
-// joined by each copy made copies of 16 MB slower than the runtime's beside a spinning OpenMP team.  Never
-// destroyed: a program may exit with contexts alive, whose threads then still wait here.
+// The threads that take part in large copies beside the calling one.  They stay until the device's last context
+// goes and are joined then: nothing of a thread outlives its contexts.  A copy does not wait for a thread that wakes
+// late (other threads of the process may keep all processors busy): it finds the job gone.  Threads started and
+// joined by each copy made copies of 16 MB slower than the runtime's beside a spinning OpenMP team.
 struct Team {
     std::thread th[kWorkers - 1];
-    int started = 0;             // guarded by g_mu
+    int started = 0;             // guarded by Pool::mu
     std::mutex mu;
     std::condition_variable wake, idle;
     Job* job = nullptr;
@@ -61,10 +55,28 @@ struct Team {
     int active = 0;
     bool stop = false;
 };
-Team& team() {
-    alignas(Team) static unsigned char place[sizeof(Team)];
-    static Team* const t = new (place) Team;
-    return *t;
+
+// What the copies of one device share.  One large copy at a time: the device's link is one, and another device's
+// copies have their own.  A copy that fits a slot goes beside a large one and does not wait for it.
+struct Pool {
+    std::mutex mu;
+    char* slots = nullptr;       // 2 * kWorkers of them
+    Team team;
+    std::mutex small_mu;
+    char* small = nullptr;       // one slot
+    std::atomic<int> users{0};   // contexts
+};
+
+// nullptr beyond the devices that have one.  Never destroyed: a program may exit with contexts alive, whose
+// threads then still wait.
+Pool* pool_of(int device) {
+    constexpr int kDevices = 64;
+    alignas(Pool) static unsigned char place[kDevices * sizeof(Pool)];
+    static Pool* const pools = [] {
+        for (int d = 0; d < kDevices; ++d) new (place + d * sizeof(Pool)) Pool;
+        return reinterpret_cast<Pool*>(place);
+    }();
+    return device >= 0 && device < kDevices ? pools + device : nullptr;
 }
 
 // Everything of the device range's chunk k that a part holds or wants, from or to the slot.
@@ -88,7 +100,7 @@ hipError_t move_device(const Job& j, size_t k, char* slot) {
 }
 
 // One thread's share: a chunk is on the link in one of its slots while it fills or empties the other.
-void work(Job& j, int w) {
+void work(Job& j, int w, char* slots) {
     auto bad = [&](hipError_t e) {
         if (e == hipSuccess) return false;
         j.error.store((int)e);
@@ -99,7 +111,7 @@ void work(Job& j, int w) {
         if (bad(hipEventCreateWithFlags(&e, hipEventDisableTiming))) break;
     size_t held[2] = {0, 0};
     bool busy[2] = {false, false};
-    auto slot = [&](int s) { return g_slots + (size_t)(2 * w + s) * kSlot; };
+    auto slot = [&](int s) { return slots + (size_t)(2 * w + s) * kSlot; };
     auto finish = [&](int s) {   // the slot's copy has ended, and what it brought is with the caller
         if (!busy[s]) return;
         busy[s] = false;
@@ -125,7 +137,8 @@ void work(Job& j, int w) {
         if (e) (void)hipEventDestroy(e);
 }
 
-void member(Team* t, int w) {
+void member(Pool* p, int w) {
+    Team* const t = &p->team;
     unsigned long long seen = 0;
     std::unique_lock<std::mutex> lk(t->mu);
     for (;;) {
@@ -137,17 +150,17 @@ void member(Team* t, int w) {
         ++t->active;
         lk.unlock();
         // (a thread that cannot take the device leaves its chunks to the others)
-        if (hipSetDevice(j.c->device) == hipSuccess) work(j, w);
+        if (hipSetDevice(j.c->device) == hipSuccess) work(j, w, p->slots);
         lk.lock();
         if (--t->active == 0) t->idle.notify_all();
     }
 }
 
-// The job by up to j.threads threads, this one among them.  g_mu is held.
-void work_together(Job& j) {
-    Team& t = team();
+// The job by up to j.threads threads, this one among them.  p->mu is held.
+void work_together(Pool* p, Job& j) {
+    Team& t = p->team;
     try {
-        for (; t.started < j.threads - 1; ++t.started) t.th[t.started] = std::thread(member, &t, t.started + 1);
+        for (; t.started < j.threads - 1; ++t.started) t.th[t.started] = std::thread(member, p, t.started + 1);
     } catch (const std::exception&) {
         // fewer threads than wanted: the others take their chunks
     }
@@ -157,15 +170,14 @@ void work_together(Job& j) {
         ++t.turn;
     }
     t.wake.notify_all();
-    work(j, 0);
+    work(j, 0, p->slots);
     std::unique_lock<std::mutex> lk(t.mu);
     t.job = nullptr;   // nobody joins any more
     t.idle.wait(lk, [&] { return t.active == 0; });
 }
 
-// g_mu is held: no copy is under way.
-void dismiss() {
-    Team& t = team();
+// No copy is under way: its lock is held.
+void dismiss(Team& t) {
     {
         std::lock_guard<std::mutex> lk(t.mu);
         t.stop = true;
@@ -188,6 +200,15 @@ struct OnDevice {
     }
 };
 
+// Memory of n bytes at p, allocated if there is none yet; false if there is none to be had.
+bool page_locked(char*& p, size_t n) {
+    if (!p && hipHostMalloc((void**)&p, n, hipHostMallocPortable) != hipSuccess) {
+        p = nullptr;
+        (void)hipGetLastError();
+    }
+    return p != nullptr;
+}
+
 int copy(lbm_ctx* c, char* dev, const HostPart* parts, int n, bool in) {
     Job j;
     j.c = c;
@@ -203,52 +224,62 @@ int copy(lbm_ctx* c, char* dev, const HostPart* parts, int n, bool in) {
     // what is queued ends before the slots are taken: others' copies do not wait for this context's steps
     HIPCHK(c, hipStreamSynchronize(c->stream));
     if (j.total == 0) return LBM_OK;
-    std::lock_guard<std::mutex> lk(g_mu);
-    if (!g_slots && hipHostMalloc((void**)&g_slots, 2 * kWorkers * kSlot, hipHostMallocPortable) != hipSuccess) {
-        // no page-locked memory: straight from and to the caller's arrays
-        g_slots = nullptr;
-        (void)hipGetLastError();
-        for (int q = 0; q < n; ++q) {
-            char* d = dev + parts[q].offset;
-            if (!parts[q].host) continue;
-            if (in) HIPCHK(c, hipMemcpyAsync(d, parts[q].host, parts[q].bytes, hipMemcpyHostToDevice, c->stream));
-            else HIPCHK(c, hipMemcpyAsync(parts[q].host, d, parts[q].bytes, hipMemcpyDeviceToHost, c->stream));
-        }
-        HIPCHK(c, hipStreamSynchronize(c->stream));
-        return LBM_OK;
-    }
     j.chunks = (j.total + kSlot - 1) / kSlot;
-    if (j.chunks == 1) {
-        if (in) move_host(j, 0, g_slots);
-        HIPCHK(c, move_device(j, 0, g_slots));
-        HIPCHK(c, hipStreamSynchronize(c->stream));
-        if (!in) move_host(j, 0, g_slots);
-        return LBM_OK;
+    Pool* const p = pool_of(c->device);
+    if (p && j.chunks == 1) {
+        std::lock_guard<std::mutex> lk(p->small_mu);
+        if (page_locked(p->small, kSlot)) {
+            if (in) move_host(j, 0, p->small);
+            HIPCHK(c, move_device(j, 0, p->small));
+            HIPCHK(c, hipStreamSynchronize(c->stream));
+            if (!in) move_host(j, 0, p->small);
+            return LBM_OK;
+        }
+    } else if (p) {
+        std::lock_guard<std::mutex> lk(p->mu);
+        if (page_locked(p->slots, 2 * kWorkers * kSlot)) {
+            // a thread costs about as much as emptying a slot: one for every two chunks
+            j.threads = (int)std::min<size_t>(kWorkers, (j.chunks + 1) / 2);
+            work_together(p, j);
+            if (j.error.load() != hipSuccess) {
+                (void)hipStreamSynchronize(c->stream);   // nothing still uses the slots
+                return hipfail(c, (hipError_t)j.error.load(), in ? "copy to the device" : "copy to the host");
+            }
+            return LBM_OK;
+        }
     }
-    // a thread costs about as much as emptying a slot: one for every two chunks
-    j.threads = (int)std::min<size_t>(kWorkers, (j.chunks + 1) / 2);
-    work_together(j);
-    if (j.error.load() != hipSuccess) {
-        (void)hipStreamSynchronize(c->stream);   // nothing still uses the slots
-        return hipfail(c, (hipError_t)j.error.load(), in ? "copy to the device" : "copy to the host");
+    // no page-locked memory: straight from and to the caller's arrays
+    for (int q = 0; q < n; ++q) {
+        char* d = dev + parts[q].offset;
+        if (!parts[q].host) continue;
+        if (in) HIPCHK(c, hipMemcpyAsync(d, parts[q].host, parts[q].bytes, hipMemcpyHostToDevice, c->stream));
+        else HIPCHK(c, hipMemcpyAsync(parts[q].host, d, parts[q].bytes, hipMemcpyDeviceToHost, c->stream));
     }
+    HIPCHK(c, hipStreamSynchronize(c->stream));
     return LBM_OK;
 }
 
 }  // namespace
 
-void transfer_retain() {
-    std::lock_guard<std::mutex> lk(g_users_mu);
-    ++g_users;
+void transfer_retain(int device) {
+    if (Pool* p = pool_of(device)) ++p->users;
 }
 
-void transfer_release() {
-    std::lock_guard<std::mutex> lk(g_users_mu);
-    if (--g_users > 0) return;
-    std::lock_guard<std::mutex> lk2(g_mu);
-    dismiss();
-    if (g_slots) (void)hipHostFree(g_slots);
-    g_slots = nullptr;
+void transfer_release(int device) {
+    Pool* const p = pool_of(device);
+    if (!p || --p->users > 0) return;
+    {
+        std::lock_guard<std::mutex> lk(p->mu);
+        if (p->users == 0) {   // (a context may have come meanwhile)
+            dismiss(p->team);
+            if (p->slots) (void)hipHostFree(p->slots);
+            p->slots = nullptr;
+        }
+    }
+    std::lock_guard<std::mutex> lk(p->small_mu);
+    if (p->users != 0) return;
+    if (p->small) (void)hipHostFree(p->small);
+    p->small = nullptr;
 }
 
 int copy_out(lbm_ctx* c, const void* dev, const HostPart* parts, int n) {

@@ -19,9 +19,9 @@ int copy_out(lbm_ctx* c, const void* dev, const HostPart* parts, int n);
 // The other way; returns when the caller's arrays have been read.  The parts cover the range.
 int copy_in(lbm_ctx* c, void* dev, const HostPart* parts, int n);
 
-// The page-locked buffers that the copies go through and the threads that take part are the process's: they come
-// with the first copy that needs them and are gone when the call for the last context returns.
-void transfer_retain();
-void transfer_release();
+// The page-locked buffers that the copies go through and the threads that take part belong to the device: they come
+// with the first copy that needs them and are gone when the call for its last context returns.
+void transfer_retain(int device);
+void transfer_release(int device);
 
 }  // namespace lbm_host

@@ -104,6 +104,12 @@ namespace {
 
 constexpr size_t kMB = 1u << 20;
 
+template <class F>
+bool until(F f) {
+    for (int n = 0; n < 2000 && !f(); ++n) std::this_thread::sleep_for(std::chrono::milliseconds(1));
+    return f();
+}
+
 std::vector<unsigned char> noise(size_t n, unsigned seed) {
     std::vector<unsigned char> v(n);
     std::mt19937_64 g(seed);
@@ -183,41 +189,81 @@ int main(int argc, char** argv) {
     lbm_ctx c;
     bool ok = false;
     if (name == "contents") {
-        transfer_retain();
+        transfer_retain(c.device);
         ok = contents(&c);
-        transfer_release();
+        transfer_release(c.device);
         ok = ok && g_locked_bytes == 0;
     } else if (name == "no_page_locked_memory") {
         g_no_lock = true;
-        transfer_retain();
+        transfer_retain(c.device);
         ok = contents(&c);
         g_no_lock = false;
         ok = ok && contents(&c);
-        transfer_release();
+        transfer_release(c.device);
     } else if (name == "errors") {
-        transfer_retain();
+        transfer_retain(c.device);
         ok = errors(&c);
-        transfer_release();
+        transfer_release(c.device);
     } else if (name == "device_of_the_caller") {
         // a context on another device than the calling thread's current one: the copies are made with its device
         // current, and the caller finds its own again
         c.device = 1;
         std::atomic<int> wrong{0};
         g_on_copy = [&](const void*, const void*, size_t) { wrong += t_device != 1; };
-        transfer_retain();
+        transfer_retain(c.device);
         ok = true;
         for (size_t n : {kMB, 20 * kMB}) {
             t_device = 0;
             ok = ok && round_trip(&c, {n}, 6, 0) && t_device == 0;
         }
-        transfer_release();
+        transfer_release(c.device);
         ok = ok && wrong == 0 && t_device == 0;
+    } else if (name == "devices_side_by_side") {
+        // two threads read out contexts on two devices: each copy waits (for a bounded time) until the other is
+        // under way
+        lbm_ctx d;
+        d.device = 1;
+        transfer_retain(c.device);
+        transfer_retain(d.device);
+        std::atomic<unsigned> seen{0};
+        std::atomic<bool> together{true};
+        g_on_copy = [&](const void*, const void*, size_t) {
+            seen |= 1u << t_device;
+            if (!until([&] { return seen == 3u; })) together = false;
+        };
+        std::atomic<int> good{0};
+        std::thread other([&] { good += round_trip(&d, {9 * kMB}, 7, 0); });
+        good += round_trip(&c, {9 * kMB}, 8, 0);
+        other.join();
+        transfer_release(c.device);
+        transfer_release(d.device);
+        ok = good == 2 && together && g_locked_bytes == 0;
+    } else if (name == "small_beside_large") {
+        // a copy of one slot ends while a large one of the same device is held up
+        transfer_retain(c.device);
+        std::atomic<bool> large{false}, small{false}, first{true};
+        g_on_copy = [&](const void*, const void*, size_t n) {
+            if (n != 2 * kMB) return;
+            large = true;
+            if (!until([&] { return small.load(); })) first = false;
+        };
+        std::atomic<int> good{0};
+        lbm_ctx d;
+        std::thread other([&] {
+            until([&] { return large.load(); });
+            good += round_trip(&d, {kMB}, 7, 0);
+            small = true;
+        });
+        good += round_trip(&c, {20 * kMB}, 8, 0);
+        other.join();
+        transfer_release(c.device);
+        ok = good == 2 && first && g_locked_bytes == 0;
     } else if (name == "threads_end") {
         // no thread that took part in a copy lives on after the last context, nor does its share of the runtime
         for (int n = 0; n < 3; ++n) {
-            transfer_retain();
+            transfer_retain(c.device);
             ok = round_trip(&c, {32 * kMB}, 5, 0);
-            transfer_release();
+            transfer_release(c.device);
             if (t_state.used) g_threads_seen = g_threads_seen.load() - 1, t_state.used = false;   // the caller's own
             ok = ok && g_threads_ended == g_threads_seen;
             if (!ok) break;
