@@ -44,6 +44,8 @@ size_t g_locked_bytes = 0;
 std::atomic<bool> g_no_lock{false};
 std::atomic<int> g_fail_after{-1};   // copies until one fails; -1: none does
 std::function<void(const void*, const void*, size_t)> g_on_copy;
+const char* g_registered = nullptr;  // the caller's memory that the runtime knows
+size_t g_registered_bytes = 0;
 
 }  // namespace
 
@@ -72,6 +74,13 @@ hipError_t hipEventRecord(hipEvent_t, hipStream_t) { return hipSuccess; }
 hipError_t hipEventSynchronize(hipEvent_t) { return hipSuccess; }
 hipError_t hipStreamSynchronize(hipStream_t) { return hipSuccess; }
 hipError_t hipGetLastError() { return hipSuccess; }
+hipError_t hipPointerGetAttributes(hipPointerAttribute_t* a, const void* p) {
+    const char* q = static_cast<const char*>(p);
+    std::memset(a, 0, sizeof *a);
+    a->type = g_registered && q >= g_registered && q < g_registered + g_registered_bytes ? hipMemoryTypeHost
+                                                                                         : hipMemoryTypeUnregistered;
+    return hipSuccess;
+}
 const char* hipGetErrorString(hipError_t) { return "an error"; }
 hipError_t hipMemcpyAsync(void* dst, const void* src, size_t n, hipMemcpyKind, hipStream_t) {
     if (g_on_copy) g_on_copy(dst, src, n);
@@ -258,6 +267,30 @@ int main(int argc, char** argv) {
         other.join();
         transfer_release(c.device);
         ok = good == 2 && first && g_locked_bytes == 0;
+    } else if (name == "arrays_the_runtime_knows") {
+        // large ones are the copies' own end, whole, whatever they stand beside; the others go through slots
+        transfer_retain(c.device);
+        ok = true;
+        for (size_t n : {kMB / 4 - 1, kMB / 4, 7 * kMB}) {
+            const int own_end = n >= kMB / 4;
+            std::vector<unsigned char> own(n), dev = noise(3 * n + 4, 9), back(dev.size()), plain(2 * n + 4);
+            g_registered = reinterpret_cast<const char*>(own.data());
+            g_registered_bytes = n;
+            const HostPart parts[4] = {{plain.data(), 0, n}, {own.data(), n, n}, {plain.data() + n, 2 * n, n},
+                                       {plain.data() + 2 * n, 3 * n, 4}};
+            std::atomic<int> direct{0}, pageable{0};
+            g_on_copy = [&](const void* to, const void* from, size_t bytes) {
+                for (const void* p : {to, from}) {
+                    if (p == own.data() && bytes == n) ++direct;
+                    if (p >= plain.data() && p < plain.data() + plain.size()) ++pageable;
+                }
+            };
+            ok = ok && copy_out(&c, dev.data(), parts, 4) == LBM_OK && direct == own_end && pageable == 0;
+            ok = ok && std::memcmp(own.data(), dev.data() + n, n) == 0 && std::memcmp(plain.data(), dev.data(), n) == 0 &&
+                 std::memcmp(plain.data() + n, dev.data() + 2 * n, n + 4) == 0;
+            ok = ok && copy_in(&c, back.data(), parts, 4) == LBM_OK && direct == 2 * own_end && pageable == 0 && back == dev;
+        }
+        transfer_release(c.device);
     } else if (name == "threads_end") {
         // no thread that took part in a copy lives on after the last context, nor does its share of the runtime
         for (int n = 0; n < 3; ++n) {
