@@ -2,13 +2,14 @@
 // other on the calling thread, which also takes the page faults of an array that is written for the
 // first time: 13-15 GB/s measured on MI355X, where the link itself carries about 50.  Here the copy
 // engine fills or empties page-locked slots while several threads do the other side.
-// Measured with 8 threads and 2 MiB slots, FP32 384x192x128: moments (154 MB) 15.6 -> 4.5 ms, a D3Q27
-// record (1.04 GB) out 97 -> 26.5 ms, in 35 -> 27 ms.  What fits one slot takes one copy on the calling
-// thread, also where it goes to several arrays (60x14x5 moments 123 -> 38 us), and spares the runtime's
-// page-locking of the caller's array on the way in (60x14x5 record 340 -> 70 us).  The first copies through a
-// new pool cost up to 2.3 ms more, as its pages are touched (equilibrium start of 112x84x70 cells, 22 MB in: 3.4
-// ms, 1.1 ms from then on; the runtime's copies 1.6 and 1.1 ms).  Slots of 1 MiB halve that, but made a readout
-// of 154 MB 0.8 ms slower.
+// Measured with 2 MiB slots, FP32 384x192x128, the runtime's copies -> these: moments (154 MB) 15.6 -> 4.2 ms, a
+// D3Q27 record (1.04 GB) out 97 -> 26.4 ms, in 35 -> 26.8 ms.  What fits one slot takes one copy on the calling
+// thread, also where it goes to several arrays (60x14x5 moments 123 -> 38 us), and spares the runtime's page-locking
+// of the caller's array on the way in (60x14x5 record 340 -> 70 us).
+// Slots are page-locked when a copy first needs them, and no more of them: at most 18 MiB a device.  The
+// equilibrium start of a program's only context of 112x84x70 cells (23 MB in, 8 MiB of slots) takes 1.9 ms and its
+// later copies 0.7 ms (the runtime's copies 1.6 and 1.1 ms; with 32 MiB at the first copy 2.0 to 3.2 ms); its first
+// moments 0.7 ms (the runtime's 1.5).  Slots of 1 MiB made a readout of 154 MB 0.8 ms slower.
 #include "transfer.h"
 
 #include <hip/hip_runtime.h>
@@ -27,7 +28,11 @@ namespace lbm_host {
 namespace {
 
 constexpr size_t kSlot = 2u << 20;   // bytes of a slot
-constexpr int kWorkers = 8;          // threads of a large copy, two slots each
+// Threads of a large copy, two slots each: one for every two chunks, as a thread costs about as much as emptying a
+// slot, up to two into the device and four out of it.  Measured on MI355X, ms with 1, 2, 4 and 8: into the device 312
+// MB 12.4, 9.1, 9.1, 9.2 (6 MB 0.32 and 0.27 with 1 and 2); out of it into new arrays, whose pages come with the first
+// write, 156 MB 13.0, 7.7, 5.0, 4.9 (into arrays that have their pages 6.1, 4.3, 4.3, 4.3).
+constexpr int kWorkers = 4, kWorkersIn = 2;
 
 struct Job {
     lbm_ctx* c;
@@ -60,7 +65,10 @@ struct Team {
 // copies have their own.  A copy that fits a slot goes beside a large one and does not wait for it.
 struct Pool {
     std::mutex mu;
-    char* slots = nullptr;       // 2 * kWorkers of them
+    char* slots[2 * kWorkers] = {};
+    int pairs = 0;               // threads that there are slots for
+    char* blocks[kWorkers] = {}; // what the slots lie in
+    int nblocks = 0;
     Team team;
     std::mutex small_mu;
     char* small = nullptr;       // one slot
@@ -99,7 +107,7 @@ hipError_t move_device(const Job& j, size_t k, char* slot) {
 }
 
 // One thread's share: a chunk is on the link in one of its slots while it fills or empties the other.
-void work(Job& j, int w, char* slots) {
+void work(Job& j, int w, char* const* slots) {
     auto bad = [&](hipError_t e) {
         if (e == hipSuccess) return false;
         j.error.store((int)e);
@@ -110,7 +118,7 @@ void work(Job& j, int w, char* slots) {
         if (bad(hipEventCreateWithFlags(&e, hipEventDisableTiming))) break;
     size_t held[2] = {0, 0};
     bool busy[2] = {false, false};
-    auto slot = [&](int s) { return slots + (size_t)(2 * w + s) * kSlot; };
+    auto slot = [&](int s) { return slots[2 * w + s]; };
     auto finish = [&](int s) {   // the slot's copy has ended, and what it brought is with the caller
         if (!busy[s]) return;
         busy[s] = false;
@@ -208,6 +216,16 @@ bool page_locked(char*& p, size_t n) {
     return p != nullptr;
 }
 
+// Threads that there are slots for, up to n; slots are added where there are fewer.  p->mu is held.
+int with_slots(Pool* p, int n) {
+    if (p->pairs < n && page_locked(p->blocks[p->nblocks], (size_t)2 * (n - p->pairs) * kSlot)) {
+        char* const b = p->blocks[p->nblocks++];
+        for (int s = 2 * p->pairs; s < 2 * n; ++s) p->slots[s] = b + (size_t)(s - 2 * p->pairs) * kSlot;
+        p->pairs = n;
+    }
+    return std::min(n, p->pairs);
+}
+
 // The parts, one at a time, straight from and to the caller's arrays.
 int straight(lbm_ctx* c, char* dev, const HostPart* parts, int n, bool in) {
     for (int q = 0; q < n; ++q) {
@@ -243,9 +261,8 @@ int staged(lbm_ctx* c, char* dev, const HostPart* parts, int n, bool in) {
         }
     } else if (p) {
         std::lock_guard<std::mutex> lk(p->mu);
-        if (page_locked(p->slots, 2 * kWorkers * kSlot)) {
-            // a thread costs about as much as emptying a slot: one for every two chunks
-            j.threads = (int)std::min<size_t>(kWorkers, (j.chunks + 1) / 2);
+        j.threads = with_slots(p, (int)std::min<size_t>(in ? kWorkersIn : kWorkers, (j.chunks + 1) / 2));
+        if (j.threads > 0) {
             work_together(p, j);
             if (j.error.load() != hipSuccess) {
                 (void)hipStreamSynchronize(c->stream);   // nothing still uses the slots
@@ -304,8 +321,11 @@ void transfer_release(int device) {
         std::lock_guard<std::mutex> lk(p->mu);
         if (p->users == 0) {   // (a context may have come meanwhile)
             dismiss(p->team);
-            if (p->slots) (void)hipHostFree(p->slots);
-            p->slots = nullptr;
+            for (; p->nblocks > 0; --p->nblocks) {
+                (void)hipHostFree(p->blocks[p->nblocks - 1]);
+                p->blocks[p->nblocks - 1] = nullptr;
+            }
+            p->pairs = 0;
         }
     }
     std::lock_guard<std::mutex> lk(p->small_mu);

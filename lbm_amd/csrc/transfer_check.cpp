@@ -291,6 +291,30 @@ int main(int argc, char** argv) {
             ok = ok && copy_in(&c, back.data(), parts, 4) == LBM_OK && direct == 2 * own_end && pageable == 0 && back == dev;
         }
         transfer_release(c.device);
+    } else if (name == "page_locked_by_need") {
+        // one slot of 2 MiB for what fits one; two slots for each thread that a larger copy takes, the same for all
+        // that follow; nothing without contexts
+        ok = true;
+        for (int rep = 0; rep < 2; ++rep) {
+            size_t locked = 0;
+            transfer_retain(c.device);
+            for (size_t n : {kMB / 10, 2 * kMB}) {
+                ok = ok && round_trip(&c, {n}, 10, 0);
+                ok = ok && g_locked_bytes <= 2 * kMB;
+            }
+            ok = ok && round_trip(&c, {3 * kMB}, 11, 0) && g_locked_bytes <= 6 * kMB;
+            ok = ok && round_trip(&c, {100 * kMB}, 12, 0);
+            locked = g_locked_bytes;
+            ok = ok && locked <= 18 * kMB && round_trip(&c, {70 * kMB, 3}, 13, 0) && g_locked_bytes == locked;
+            transfer_release(c.device);
+            ok = ok && g_locked_bytes == 0;
+        }
+        // into the device only
+        std::vector<unsigned char> to(22 * kMB), from = noise(to.size(), 14);
+        const HostPart part{from.data(), 0, from.size()};
+        transfer_retain(c.device);
+        ok = ok && copy_in(&c, to.data(), &part, 1) == LBM_OK && to == from && g_locked_bytes <= 8 * kMB;
+        transfer_release(c.device);
     } else if (name == "threads_end") {
         // no thread that took part in a copy lives on after the last context, nor does its share of the runtime
         for (int n = 0; n < 3; ++n) {

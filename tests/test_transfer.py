@@ -10,7 +10,8 @@ EXE = os.path.join(ROOT, "lbm_amd", "_build", "transfer_check")
 
 
 @pytest.mark.parametrize("case", ["contents", "no_page_locked_memory", "errors", "threads_end", "device_of_the_caller",
-                                  "devices_side_by_side", "small_beside_large", "arrays_the_runtime_knows"])
+                                  "devices_side_by_side", "small_beside_large", "arrays_the_runtime_knows",
+                                  "page_locked_by_need"])
 def test_transfer(case):
     if not os.path.exists(EXE):
         pytest.fail("transfer_check not built (python -m lbm_amd.build)")
