@@ -258,11 +258,12 @@ int lbm_adjoint_run(lbm_ctx* c, int it0, int nsteps, int every, const int32_t* b
         std::vector<double> hs((size_t)d.ny * d.nz), ha(2 * (size_t)nblk);
         const size_t gbytes = 3 * ncell_padded(c) * sizeof(double);
         if (gFp) {
-            // the gradient in the reference's layout
-            if (int r = dev_alloc(c, c->stage, gbytes)) return r;
-            HIPCHK(c, (cells_out<3, true>(c->lay, GradientOut{gFp}, static_cast<double*>(c->stage.p), c->stream)));
+            // the gradient in the reference's layout, turned in the adjoint buffers, which have done their work (2 * q
+            // populations of 4 bytes a cell at least, 24 bytes here): nothing is allocated after the forward sweep
+            double* const turned = static_cast<double*>(lam.p);
+            HIPCHK(c, (cells_out<3, true>(c->lay, GradientOut{gFp}, turned, c->stream)));
             const HostPart part{grad_force, 0, gbytes};
-            if (int r = copy_out(c, c->stage.p, &part, 1)) return r;
+            if (int r = copy_out(c, turned, &part, 1)) return r;
         }
         HIPCHK(c, hipMemcpyAsync(ha.data(), acc.p, ha.size() * sizeof(double), hipMemcpyDeviceToHost, c->stream));
         HIPCHK(c, hipMemcpyAsync(hs.data(), gS.p, hs.size() * sizeof(double), hipMemcpyDeviceToHost, c->stream));
