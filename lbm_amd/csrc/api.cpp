@@ -217,6 +217,22 @@ EdgeList edge_list(const lbm_desc& d) {
     return e;
 }
 
+// Whether the step kernel of a duct (two closed axes) writes the inflow/outflow planes but for their rows along the
+// walls.  That takes most of the launch behind the step, but a row's two ends store to scattered lines at the end of
+// their wave's time.  Measured on MI355X over 438 ducts (D3Q19 and D3Q27, 16 <= nx <= 300, planes of 2745 to 30000
+// cells of 12x500 to 300x16), time of a step with separate planes / with planes in the step:
+//   planes below 64x64: 0.86-1.07; of 64x64: D3Q27 FP32 0.99-1.04, the others 0.80-1.02;
+//   32-bit storage, larger planes: 0.98-1.50, but for D3Q19 planes below 6500 cells (0.86-1.11, the half of them gain);
+//   16-bit, rows of one wave (nx <= 64, both ends in it): 0.74-1.04 below 14400 cells, 0.94-1.53 from there on; longer
+//   rows: 0.99-1.46;
+//   64-bit: 0.91-1.33 up to nx = 160 (below 1 at nx = 90 only), 0.95-1.01 beyond.
+bool inflow_in_step(int raw_bytes, const lbm_desc& d) {
+    const long long plane = (long long)d.ny * d.nz;
+    if (raw_bytes == 4) return plane >= 4096;
+    if (raw_bytes == 2 && d.nx <= 64) return plane >= 14400;
+    return plane > 4096 && (raw_bytes == 2 || d.nx <= 160);
+}
+
 double utime_at(const lbm_ctx* c, int it) {
     if (!c->ut_series.empty() && it >= c->series_lo && it <= c->series_hi) return c->ut_series[it - c->series_lo];
     return c->uini;
@@ -459,15 +475,11 @@ int lbm_create(const lbm_desc* desc, lbm_ctx** out) {
     // storage axes mapped at run time.
     if (const char* v = getenv("LBM_STEP_VARIANT")) c->variant = atoi(v) & 7;
     {
-        // With one closed axis (no edges, corners or snapshots then) the step kernel can perform
-        // that axis's face pass itself, and with at most that one closed axis the inflow/outflow
-        // planes of i as well: a step is then one launch.  With two closed axes the inflow/outflow planes
-        // are the step kernel's but for the rows along the walls, from planes of 4096 cells on: measured on
-        // MI355X, FP32, separate -> in the step, us per step: D3Q27 250x98x70 90.1 -> 84.0, 60x150x120
-        // 89.8 -> 62.8, 300x150x90 197 -> 192, but 100x61x45 26.7 -> 25.9 (D3Q19 19.7 -> 20.6) and 30x16x14
-        // 8.8 -> 11.0, where the scattered stores at the end of a wave are the step's latency; FP16 alike,
-        // FP64 -1 to +12 %.  Ensembles always fold the face (a member's face must not need a launch of its
-        // own).  LBM_FOLD=0 selects the separate boundary kernel for a single domain.
+        // With one closed axis (no edges or corners then) the step kernel can perform that axis's face pass itself,
+        // and with at most that one closed axis the inflow/outflow planes of i as well: a step is then one launch.
+        // With two closed axes the inflow/outflow planes are the step kernel's but for the rows along the walls, where
+        // inflow_in_step says so.  Ensembles always fold the face (a member's face must not need a launch of
+        // its own).  LBM_FOLD=0 selects the separate boundary kernel for a single domain.
         const int codes[3] = {d.ibnd, d.jbnd, d.kbnd};
         int nclosed = 0, cl = -1;
         for (int a = 0; a < 3; ++a)
@@ -477,8 +489,7 @@ int lbm_create(const lbm_desc* desc, lbm_ctx** out) {
         // halo domains always fold: the separate boundary kernels do not know halo planes
         const bool fold = d.jbnd == LBM_BND_HALO || (fv ? atoi(fv) != 0 : kFoldDefault);
         c->fold_on = c->fold_dir >= 0 && fold;
-        const bool wide = (long long)d.ny * d.nz >= 4096;
-        c->inflow_fold_on = d.ibnd != 1 || !fold ? 0 : nclosed < 2 ? 1 : wide ? 2 : 0;
+        c->inflow_fold_on = d.ibnd != 1 || !fold ? 0 : nclosed < 2 ? 1 : inflow_in_step(ops->raw_bytes, d) ? 2 : 0;
         // LBM_INFLOW_FOLD=0 keeps the face folded but writes the inflow/outflow planes with their own
         // kernel (measured slower: tile 384x24x128 14.0 k vs 16.2 k MLUPS, whole domain -1 %)
         // LBM_INFLOW_FOLD=1 folds them with two closed axes whatever the size
