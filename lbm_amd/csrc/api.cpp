@@ -504,7 +504,7 @@ int lbm_create(const lbm_desc* desc, lbm_ctx** out) {
     scratch_resolve(c->device);
     // Resident step-kernel blocks per CU, capped by reserving 1/n of the CU's LDS per block (the
     // kernel itself uses none).  D3Q27 with 4-byte storage: 5 waves per SIMD (20 per CU; 5 blocks of
-    // 64 x 4 cells) where its 78 VGPRs would allow 6 (measured on MI355X, reg+Vreman 384x192x128:
+    // 64 x 4 cells) where its 73 VGPRs would allow 6 (measured on MI355X at 78, reg+Vreman 384x192x128:
     // 351.1 us per step kernel against 358.9 us; 768x256x192: 1373 us against 1444 us); the 16-bit
     // and D3Q19 kernels run best uncapped.  LBM_STEP_BLOCKS_PER_CU=n overrides (0: no cap).
     {

@@ -901,10 +901,10 @@ __device__ __forceinline__ void st(const Layout& L, void* f, int l, int off, typ
 //     call, which the thread that replaces it passes on first;
 //   * S on an inflow plane and a closed axis at once: no pass writes it.
 // Measured on MI355X, FP32, per step: closed box 101x61x45 (three closed axes) 38.4 us in four launches
-// -> 7.9 us; duct 250x98x70 (inflow, two closed axes) 52.1 us in four launches -> 25.5 us.  The inflow planes
-// were most of the duct's: with i contiguous, four lines for every value.  Now the step kernel's end cells
-// write them but for the rows along the walls (inflow_fold = 2), and the launch takes 11.6 us; the
-// two kernels of a step 92 -> 89.5 us.
+// -> 7.9 us; duct 250x98x70 (inflow, two closed axes) 52.1 us in four launches -> 25.5 us (a kernel trace, which
+// runs launches apart).  The inflow planes were most of the duct's: with i contiguous, four lines for every value.
+// Where the step kernel's end cells write them but for the rows along the walls (inflow_fold = 2), the launch
+// takes 11.6 us and the step kernel 78 instead of 66 us in the trace; untraced a step takes 84 us instead of 90.
 template <int Q, class C>
 __global__ void __launch_bounds__(256) boundary_kernel(const BoundaryArgs<typename C::real> a) {
     using R = typename C::real;
@@ -1190,9 +1190,9 @@ __global__ void __launch_bounds__(256) halo_unpack_kernel(Layout L, void* f, int
 
 // ------------------------------------------------------------------------------------------
 // Ensembles: many domains of one lattice, storage and collision model advanced by one launch of
-// a persistent kernel per step.  Every domain's rows are cut into segments of 64 bytes, and the
+// a kernel per step.  Every domain's rows are cut into segments of 64 bytes, and the
 // segments of each (ax0, ax1) plane into tiles of blockDim.x cells; the tiles of all members form one
-// list that the blocks of the grid walk with stride gridDim.x.  Whole segments matter: tiles of
+// list that the blocks of the grid walk with stride gridDim.x (by default a block for each).  Whole segments matter: tiles of
 // consecutive cells, which the first form cut regardless of rows, left lines of rows that are no
 // multiple of 64 cells to two waves, whose separate partial stores memory read and wrote twice.
 // Measured on MI355X, D3Q19 per step: 16 members of about 112x84x70 cells (10.8 M) FP32 560 -> 319 us,

@@ -6,7 +6,7 @@
 // D3Q27 record (1.04 GB) out 97 -> 26.4 ms, in 35 -> 26.8 ms.  What fits one slot takes one copy on the calling
 // thread, also where it goes to several arrays (60x14x5 moments 123 -> 38 us), and spares the runtime's page-locking
 // of the caller's array on the way in (60x14x5 record 340 -> 70 us).
-// Slots are page-locked when a copy first needs them, and no more of them: at most 18 MiB a device.  The
+// Slots are page-locked when a copy first needs them, and no more of them: at most 22 MiB a device.  The
 // equilibrium start of a program's only context of 112x84x70 cells (23 MB in, 8 MiB of slots) takes 1.9 ms and its
 // later copies 0.7 ms (the runtime's copies 1.6 and 1.1 ms; with 32 MiB at the first copy 2.0 to 3.2 ms); its first
 // moments 0.7 ms (the runtime's 1.5).  Slots of 1 MiB made a readout of 154 MB 0.8 ms slower.
@@ -29,10 +29,11 @@ namespace {
 
 constexpr size_t kSlot = 2u << 20;   // bytes of a slot
 // Threads of a large copy, two slots each: one for every two chunks, as a thread costs about as much as emptying a
-// slot, up to two into the device and four out of it.  Measured on MI355X, ms with 1, 2, 4 and 8: into the device 312
-// MB 12.4, 9.1, 9.1, 9.2 (6 MB 0.32 and 0.27 with 1 and 2); out of it into new arrays, whose pages come with the first
-// write, 156 MB 13.0, 7.7, 5.0, 4.9 (into arrays that have their pages 6.1, 4.3, 4.3, 4.3).
-constexpr int kWorkers = 4, kWorkersIn = 2;
+// slot, up to two into the device and five out of it.  Measured on MI355X, ms with 1, 2, 4, 5 and 8: into the device
+// 312 MB 12.4, 9.1, 9.1, 9.2, 9.2 (6 MB 0.32 and 0.27 with 1 and 2); out of it into new arrays, whose pages come with
+// the first write, 156 MB 13.0, 7.7, 4.9, 4.8, 4.9 (into arrays that have their pages 6.1, 4.3, 4.3, 4.3, 4.3), 1.04 GB
+// 26.5, 26.4, 26.5 with 4, 5 and 8 (32 with 3).
+constexpr int kWorkers = 5, kWorkersIn = 2;
 
 struct Job {
     lbm_ctx* c;

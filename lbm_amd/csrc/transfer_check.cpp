@@ -305,7 +305,7 @@ int main(int argc, char** argv) {
             ok = ok && round_trip(&c, {3 * kMB}, 11, 0) && g_locked_bytes <= 6 * kMB;
             ok = ok && round_trip(&c, {100 * kMB}, 12, 0);
             locked = g_locked_bytes;
-            ok = ok && locked <= 18 * kMB && round_trip(&c, {70 * kMB, 3}, 13, 0) && g_locked_bytes == locked;
+            ok = ok && locked <= 22 * kMB && round_trip(&c, {70 * kMB, 3}, 13, 0) && g_locked_bytes == locked;
             transfer_release(c.device);
             ok = ok && g_locked_bytes == 0;
         }
