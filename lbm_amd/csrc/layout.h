@@ -2,7 +2,7 @@
 //
 // Cells of the padded grid (0:nx+1, 0:ny+1, 0:nz+1) lie in rows along one axis (the "fast" axis);
 // interior index 1 starts on a 128-byte boundary and the row pitch is the smallest multiple of 128
-// bytes that holds a row's n + 2 cells.  Ghost 0 of a row is the last element of the row before it
+// bytes that holds a row's n + 2 cells, or one more (row_lines).  Ghost 0 of a row is the last element of the row before it
 // (behind that row's ghost n + 1); one line before the first row holds the first row's.  A line of
 // its own for that one ghost (the pitch before) left a quarter of the buffer's 256-byte blocks
 // untouched at 192 cells of 4 bytes and a third at 96; measured on MI355X with the smaller pitch,
@@ -90,6 +90,27 @@ __host__ __device__ inline int part_row(int c, int part, int n, int e) {
 // Elements of a 128-byte line.
 __host__ __device__ inline constexpr int line_elems(int raw_bytes) { return 128 / raw_bytes; }
 
+// Lines of a row of n0 cells of a domain of `rows` rows and nq populations (0: per-cell arrays only).  The least that
+// holds them and both ghosts, but where the row's axis is periodic
+//   * no power of two from 8 lines on (16-bit storage from 16, D3Q27 FP32 up to 16), at which the populations of a cell
+//     lie on few of the memory's channels.  Measured on MI355X, step with the least / with one line more, grids of 1.5 to
+//     9 M cells: FP32 8 lines (223 to 254 cells) 1.03-1.06, 16 lines 1.01-1.09, D3Q19 32 lines 1.03-1.05 (D3Q27 0.98);
+//     FP64 8, 16 and 32 lines 1.00-1.04; FP16 16 and 32 lines 1.00-1.04, 8 lines 0.98-1.00; 4 lines 0.97-1.03.
+//   * 26 and 28 lines for 25 and 27 (FP32), whole 256-byte blocks, in buffers that the 256 MB of last-level cache do not
+//     hold: D3Q19 25 lines (767 to 798 cells) 1.00-1.07 (768x256x192 970 -> 948 us), 27 lines 1.03-1.09, D3Q27 1.00.  Smaller
+//     buffers lose up to 2.5 %; longer odd rows (29 to 35 lines) 0.97-1.04, shorter ones (7 to 23) 0.94-1.01, FP64 rows
+//     0.97-1.00.
+// Rows along a closed or an inflow axis keep the least: a line more puts ghost 0 into a line that holds nothing else (duct
+// 250x98x70, FP32, 84.5 -> 88.2 us).
+inline int row_lines(int n0, int raw_bytes, int nq, double rows, bool periodic) {
+    const int a = line_elems(raw_bytes), n = (n0 + 2 + a - 1) / a;
+    auto power = [](int v) { return (v & (v - 1)) == 0; };
+    if (!periodic || raw_bytes > 8) return n;
+    if (power(n) && n >= (raw_bytes == 2 ? 16 : 8) && n <= (raw_bytes == 4 && nq == 27 ? 16 : 32)) return n + 1;
+    if (raw_bytes == 4 && (n == 25 || n == 27) && rows * nq * n * 128.0 > 268435456.0) return n + 1;
+    return n;
+}
+
 // fast < 0: choose (first periodic axis, else i).  q > 0 with rowblock: row-blocked buffers when every
 // element offset fits 31 bits and one slab of the slowest axis (Q rows per ax1 index) and the line
 // behind it stay below 4 GiB (the step kernel's 32-bit offsets within a slab), planes otherwise.
@@ -104,7 +125,8 @@ inline Layout make_layout(int nx, int ny, int nz, int raw_bytes, int per_i, int 
     L.ax2 = fast == 2 ? 1 : 2;
     const int a = line_elems(raw_bytes);
     const int n0 = L.n(L.ax0), n1 = L.n(L.ax1), n2 = L.n(L.ax2);
-    L.pitch = (n0 + 2 + a - 1) / a * a;
+    const bool per0 = fast == 0 ? per_i : fast == 1 ? per_j : per_k;
+    L.pitch = row_lines(n0, raw_bytes, q, (n1 + 2.0) * (n2 + 2.0), per0) * a;
     int st[3];
     st[L.ax0] = 1;
     st[L.ax1] = L.pitch;

@@ -12,6 +12,7 @@
 //     and map every other launch coordinate past the last cell, for any block height.
 // Prints one JSON line per case; exits non-zero on the first violation.
 #include <cstdio>
+#include <cstring>
 #include <cstdlib>
 #include <vector>
 
@@ -80,7 +81,44 @@ static int check(int nx, int ny, int nz, int raw, int q, int pi, int pj, int pk,
     return 0;
 }
 
-int main() {
+// Row pitches (row_lines): the layouts of rows at and next to the lengths where a line is added, as above; what the
+// pitch is for rows of every length.
+static int check_rows(int* n) {
+    for (int raw : {2, 4, 8})
+        for (int q : {19, 27})
+            for (int lines : {4, 8, 9, 16, 24, 25, 32})
+                for (int off : {-1, 0, 1})
+                    for (int axis = 0; axis < 3; ++axis)
+                        for (int per : {0, 1}) {
+                            const int n0 = lines * line_elems(raw) - 2 + off;
+                            const int d[3] = {axis == 0 ? n0 : 3, axis == 1 ? n0 : 3, axis == 2 ? n0 : 2};
+                            const int p[3] = {axis == 0 ? per : 0, axis == 1 ? per : 0, axis == 2 ? per : 0};
+                            for (int rb = 0; rb < 2; ++rb)
+                                if (const int rc = check(d[0], d[1], d[2], raw, q, p[0], p[1], p[2], rb != 0, axis)) return rc;
+                            ++*n;
+                        }
+    for (int raw : {2, 4, 8, 16})
+        for (int q : {0, 19, 27})
+            for (int per : {0, 1})
+                for (int n0 = 2; n0 < 5000; ++n0)
+                    for (double rows : {100.0, 50000.0}) {
+                        const int a = line_elems(raw), least = (n0 + 2 + a - 1) / a, l = row_lines(n0, raw, q, rows, per != 0);
+                        if (l < least || l > least + 1 || (l != least && (!per || raw == 16 || least < 8))) return 13;
+                        if (per && raw == 4 && (l == 8 || l == 16 || (l == 32 && q != 27))) return 14;
+                        if (per && raw == 8 && (l == 8 || l == 16 || l == 32)) return 14;
+                        if (per && raw == 4 && q == 19 && least == 25 && l != (rows > 1000 ? 26 : 25)) return 15;
+                        ++*n;
+                    }
+    return 0;
+}
+
+int main(int argc, char** argv) {
+    if (argc > 1 && std::strcmp(argv[1], "rows") == 0) {
+        int n = 0;
+        const int rc = check_rows(&n);
+        std::printf("{\"rows\": %d, \"error\": %d}\n", n, rc);
+        return rc;
+    }
     const int dims[][3] = {{20, 14, 12}, {18, 13, 10}, {12, 8, 6}, {64, 24, 12}, {96, 32, 16}, {7, 5, 3}};
     const int pers[][3] = {{0, 1, 0}, {1, 0, 0}, {0, 0, 1}, {0, 0, 0}, {1, 1, 1}};
     int n = 0;
