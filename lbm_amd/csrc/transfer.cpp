@@ -311,6 +311,13 @@ int copy(lbm_ctx* c, char* dev, const HostPart* parts, int n, bool in) {
 
 }  // namespace
 
+HostResults::HostResults(const lbm_ctx* c) {
+    Pool* const pool = pool_of(c->device);
+    if (!pool) return;
+    lock = std::unique_lock<std::mutex>(pool->small_mu);
+    if (page_locked(pool->small, kSlot)) p = pool->small;
+}
+
 void transfer_retain(int device) {
     if (Pool* p = pool_of(device)) ++p->users;
 }
