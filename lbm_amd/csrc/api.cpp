@@ -901,16 +901,25 @@ int lbm_set_blanking(lbm_ctx* c, const uint8_t* mask) {
     const int wpr = (n0 + 31) / 32;
     std::vector<uint32_t> bits((size_t)wpr * n1 * n2, 0u);
     bool any = false;
+    const size_t step[3] = {1, (size_t)d.nx + 2, (size_t)(d.nx + 2) * (d.ny + 2)};   // of the mask along i, j, k
+    const size_t s = step[L.ax0];
+    auto word_of = [](const uint8_t* m, size_t st, int n) {
+        uint32_t v = 0;
+        for (int b = 0; b < n; ++b) v |= (uint32_t)(m[b * st] != 0) << b;
+        return v;
+    };
+    uint32_t* word = bits.data();
+    uint32_t seen = 0;
     for (int cc = 1; cc <= n2; ++cc)
-        for (int cb = 1; cb <= n1; ++cb)
-            for (int ca = 1; ca <= n0; ++ca) {
-                int i, j, k;
-                L.ijk(ca, cb, cc, i, j, k);
-                if (mask[((size_t)k * (d.ny + 2) + j) * (d.nx + 2) + i]) {
-                    bits[((size_t)(cc - 1) * n1 + (cb - 1)) * wpr + (ca - 1) / 32] |= 1u << ((ca - 1) % 32);
-                    any = true;
-                }
+        for (int cb = 1; cb <= n1; ++cb) {
+            const uint8_t* m = mask + cc * step[L.ax2] + cb * step[L.ax1] + s;
+            for (int w = 0; w < wpr; ++w, m += 32 * s) {
+                const int n = std::min(32, n0 - 32 * w);
+                *word = n < 32 ? word_of(m, s, n) : s == 1 ? word_of(m, 1, 32) : word_of(m, s, 32);
+                seen |= *word++;
             }
+        }
+    any = seen != 0;
     if (int rc = dev_alloc(c, c->solid, bits.size() * 4)) return rc;
     HIPCHK(c, hipMemcpyAsync(c->solid.p, bits.data(), bits.size() * 4, hipMemcpyHostToDevice, c->stream));
     HIPCHK(c, hipStreamSynchronize(c->stream));
